@@ -228,3 +228,24 @@ def test_dense_a8_vec(dev, t, tokens):
     scale = np.abs(ref).max()
     assert np.abs(got - ref).max() <= 1e-2 * scale + 1e-6, (np.abs(got - ref).max(), scale)
     assert R.rel_errors(got, ref)[0] < 5e-3
+
+
+@pytest.mark.parametrize("n,E", [(1024, 256), (1025, 256), (4097, 512), (131077, 4000)])
+def test_hot_route_counts_of_long_calls(dev, n, E):
+    """The per-route counts (up to 1024 routes) and the LDS counts above, past a block's 4096
+    routes and with expert ids past the LDS bins: a popular expert on half of the routes,
+    counts added to what is there."""
+    import torch
+
+    *_, C = _pkg()
+    rng = np.random.default_rng(n)
+    ids = np.where(rng.random(n) < 0.5, E - 1, rng.integers(0, E, n)).astype(np.int32)
+    log2slot = np.where(rng.random(E) < 0.2, rng.integers(0, 64, E), -1).astype(np.int32)
+    log2cpu = np.where(log2slot >= 0, -1, np.arange(E)).astype(np.int32)
+    before = rng.integers(0, 1000, E).astype(np.float32)
+    counts = to_dev(before, dev)
+    s, c = C.route_native(to_dev(ids, dev), to_dev(log2slot, dev), to_dev(log2cpu, dev), counts)
+    torch.cuda.synchronize()
+    assert np.array_equal(s.cpu().numpy(), log2slot[ids]) and np.array_equal(c.cpu().numpy(), log2cpu[ids])
+    assert np.array_equal(counts.cpu().numpy(), before + np.bincount(ids, minlength=E).astype(np.float32))
+
