@@ -2,6 +2,8 @@
 // grouped GEMMs' decoder), the hot
 // cache's route lookup, q8_1 activation quantisation, SiLU*mul and the weighted top-k
 // combine.
+#include <type_traits>
+
 #include "bpiece.h"
 #include "kernels.h"
 
@@ -9,32 +11,20 @@ namespace ktmi {
 
 // ---------------------------------------------------------------- dequant
 // The grouped GEMMs' own decoder (bpiece.h) run stand-alone, so the bytes-to-bf16 step the
-// GEMMs feed to the matrix cores is the one this entry point exposes (and its tests pin):
-// the same lane -> (row, half) map (lane % 32 = row of a 32-row group, lane / 32 = half h
-// of a 64-value step), the same load_head / load<SUB> / decode<SUB> calls. Each wave runs
-// 32 rows over the 4 steps of one 256-value super-block column and writes every decoded
-// 8-value chunk (16 bytes) to its K position 256 sb + ksub<SUB>() + coff(q).
-// grid (ceil(row groups x columns / 4), n); P:11471-11498 contract, all four formats.
-template <int TYPE, int SUB>
-__device__ __forceinline__ void dequant_step(const uint8_t* row, int sb, int h, int64_t cols,
-                                             const typename BPiece<TYPE>::Head& hd, const uint32_t* grid,
-                                             uint16_t* orow) {
-  using BP = BPiece<TYPE>;
-  const int64_t k0 = 256 * (int64_t)sb + BP::template ksub<SUB>();
-  // Q8_0 rows may end inside a super-block column (a piece is one 32-value block): the
-  // pieces past the row's end are not loaded
-  if (k0 + BP::off0(h) >= cols) return;
-  typename BP::Raw raw;
-  uint32_t v[16];
-  BP::template load<SUB>(row, sb, h, grid, raw);
-  BP::template decode<SUB>(hd, raw, grid, v);
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int pos = (c < 2 ? BP::off0(h) : BP::off1(h)) + 8 * (c & 1);  // step position of chunk c
-    const u32x4_t w = {v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]};
-    *(u32x4_t*)(orow + k0 + BP::coff(pos / 8)) = w;
-  }
-}
+// GEMMs feed to the matrix cores is the one this entry point exposes (and its tests pin): the
+// same load_head / load / decode bodies, half h = lane / 32 of a 64-value step as there.
+// P:11471-11498 contract, all four formats.
+//
+// Bound by HBM: a value is read as half a byte to a byte and written as two. A wave takes 16
+// consecutive (row, 256-value column) units, four lanes (step parity p, half h) to a unit, so
+// the raw bytes of a wave are one contiguous range and so is its output; each lane's decoded
+// chunks (16 bytes, 64 to 192 bytes apart) pass through LDS, where the wave picks them up in
+// memory order: every store instruction writes whole 256-byte segments. With a lane to a row
+// and the chunks stored straight from the registers, an instruction touched 64 segments and
+// eight 7168 x 2048 Q6_K experts took 144 us (2.3 TB/s); so they take 67 us (4.9 TB/s,
+// the rate of a large copy on this card).
+constexpr int DQ_UNITS = 16;                      // (row, column) units a wave
+constexpr int DQ_STG = DQ_UNITS * 256;            // staging bytes a wave: 128 bf16 values a unit
 
 template <int TYPE>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ raw, int64_t raw_stride,
@@ -42,32 +32,74 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
                                                       uint16_t* __restrict__ out, int64_t out_stride) {
   using BP = BPiece<TYPE>;
   __shared__ uint32_t grid[TYPE == GGML_IQ3_S ? 512 : 1];
+  __shared__ __attribute__((aligned(16))) uint8_t stage[4 * DQ_STG];
   if constexpr (TYPE == GGML_IQ3_S) {
     stage_iq3s_sel(grid);
     __syncthreads();
   }
   const int64_t e = blockIdx.y;
-  const int lane = threadIdx.x & 63, h = lane >> 5;
-  const int64_t nsb = (cols + 255) / 256;
-  const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // (row group, column)
-  if (unit >= (rows + 31) / 32 * nsb) return;
-  const int64_t r = unit / nsb * 32 + (lane & 31);
-  const int sb = (int)(unit % nsb);
-  if (r >= rows) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p = lane & 1, h = lane >> 5, ul = (lane & 31) >> 1;
+  const int64_t nsb = (cols + 255) / 256, total = rows * nsb;
+  const int64_t u0 = ((int64_t)blockIdx.x * 4 + wave) * DQ_UNITS;  // the wave's first unit
+  if (u0 >= total) return;
+  const int64_t r0 = u0 / nsb;
+  const uint32_t sb0 = (uint32_t)(u0 - r0 * nsb);
+  // row and column of the wave's unit q
+  auto place = [&](int q, int64_t& r, int& sb) {
+    const uint32_t t = sb0 + (uint32_t)q, dr = t / (uint32_t)nsb;
+    r = r0 + dr;
+    sb = (int)(t - dr * (uint32_t)nsb);
+  };
+  int64_t r;
+  int sb;
+  place(ul, r, sb);
   const uint8_t* row = raw + e * raw_stride + r * rb;
-  uint16_t* orow = out + e * out_stride + r * cols;
+  const bool live = u0 + ul < total;
   typename BP::Head hd;
-  BP::load_head(row, sb, h, hd);
-  dequant_step<TYPE, 0>(row, sb, h, cols, hd, grid, orow);
-  dequant_step<TYPE, 1>(row, sb, h, cols, hd, grid, orow);
-  dequant_step<TYPE, 2>(row, sb, h, cols, hd, grid, orow);
-  dequant_step<TYPE, 3>(row, sb, h, cols, hd, grid, orow);
+  typename BP::Raw rw[2];
+  // Q8_0 rows may end inside a column (a piece is one 32-value block): the pieces past the
+  // row's end are not loaded
+  auto inside = [&](int ks) { return live && 256 * (int64_t)sb + ks + BP::off0(h) < cols; };
+  if (live) BP::load_head(row, sb, h, hd);
+  if (inside(BP::template ksub_hp<0>(p))) BP::template load_hp<0>(row, sb, h, p, grid, rw[0]);
+  if (inside(BP::template ksub_hp<1>(p))) BP::template load_hp<1>(row, sb, h, p, grid, rw[1]);
+  uint8_t* stg = stage + wave * DQ_STG;
+  uint16_t* oe = out + e * out_stride;
+  auto half = [&](auto s2c) {
+    constexpr int S2 = decltype(s2c)::value;
+    uint32_t v[16];
+    BP::template decode_hp<S2>(hd, rw[S2], grid, p, v);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int q = c < 2 ? BP::off0(h) / 8 + c : BP::off1(h) / 8 + c - 2;
+      const int slot = (BP::template ksub_hp<S2>(p) - 128 * S2 + BP::coff(q)) / 8;  // 16-byte slot of the unit
+      const u32x4_t w = {v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]};
+      *(u32x4_t*)(stg + ul * 256 + 16 * (slot ^ ul)) = w;  // slot ^ unit: no bank conflicts
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const int q = 4 * it + (lane >> 4), slot = lane & 15;
+      const u32x4_t w = *(const u32x4_t*)(stg + q * 256 + 16 * (slot ^ q));
+      int64_t qr;
+      int qs;
+      place(q, qr, qs);
+      const int64_t k = 256 * (int64_t)qs + 128 * S2 + 8 * slot;
+      if (u0 + q < total && k < cols) __builtin_nontemporal_store(w, (u32x4_t*)(oe + qr * cols + k));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  half(std::integral_constant<int, 0>{});
+  half(std::integral_constant<int, 1>{});
 }
 
 int launch_dequant(const uint8_t* raw, int64_t raw_stride, int type, int64_t n, int64_t rows, int64_t cols,
                    uint16_t* out, int64_t out_stride, hipStream_t stream) {
-  const int64_t units = (rows + 31) / 32 * ((cols + 255) / 256);
-  dim3 grid((unsigned)((units + 3) / 4), (unsigned)n);
+  const int64_t units = rows * ((cols + 255) / 256);
+  dim3 grid((unsigned)((units + 4 * DQ_UNITS - 1) / (4 * DQ_UNITS)), (unsigned)n);
   const int64_t rb = row_bytes(cols, type);
   switch (type) {
     case GGML_Q8_0: dequant_kernel<GGML_Q8_0><<<grid, 256, 0, stream>>>(raw, raw_stride, rows, cols, rb, out, out_stride); break;

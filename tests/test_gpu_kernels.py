@@ -249,3 +249,25 @@ def test_hot_route_counts_of_long_calls(dev, n, E):
     assert np.array_equal(s.cpu().numpy(), log2slot[ids]) and np.array_equal(c.cpu().numpy(), log2cpu[ids])
     assert np.array_equal(counts.cpu().numpy(), before + np.bincount(ids, minlength=E).astype(np.float32))
 
+
+@pytest.mark.parametrize("t", TYPES)
+def test_dequant_wave_edges(dev, t):
+    """A wave's 16 (row, column) units: fewer than one wave's, a unit past it, rows whose
+    columns straddle waves, and (Q8_0) rows that end inside a column."""
+    import torch
+
+    DQ, *_ = _pkg()
+    rng = np.random.default_rng(500 + t)
+    shapes = [(1, 256), (17, 256), (5, 768), (67, 1280)] + ([(3, 32), (19, 1056)] if t == R.GGML_Q8_0 else [])
+    for rows, cols in shapes:
+        raw = np.stack([random_blocks(t, rows, cols, rng).reshape(-1) for _ in range(2)])
+        raw = np.pad(raw, ((0, 0), (0, -raw.shape[1] % 16)))
+        out = torch.full((2, (rows * cols + 7) // 8 * 8 + 64), -1, dtype=torch.int16, device=dev).view(torch.bfloat16)
+        view = out[:, :rows * cols].view(2, rows, cols)
+        DQ.dequant_experts(to_dev(raw, dev), raw.shape[1], t, 2, rows, cols, view)
+        torch.cuda.synchronize()
+        got = bf16_bits_of(out)
+        n = rows * R.row_bytes(cols, t)
+        for e in range(2):
+            assert np.array_equal(got[e, :rows * cols], R.dequant_experts(raw[e, :n], t, 1, rows, cols).reshape(-1)), (rows, cols)
+            assert np.all(got[e, rows * cols:] == 0xFFFF), "wrote past the expert"
