@@ -186,12 +186,14 @@ static int scratch_of_current_device(void** out) {
 // (graph-replayed steps of the 2048 x 512 Q4_K layer with 32 hot slots: 13.0 against 15.0 us at
 // 8 routes, 19.5 against 19.2 at 32); from 64 routes the decode mode's MFMAs win (23.0 against
 // 25.8 at 64, 24.2 against 30.9 at 128).
+// Where the rows are too long for those two launches, the decode mode starts at one route: its
+// alternative is the stage-by-stage GEMV (7168 x 2048 Q4_K/Q6_K, 40 routes: 189-244 against 87 us).
 constexpr int64_t kDecodeMinRoutes = 64;
 
 int ktmi_moe_layer_mode(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
   if (tokens * top_k > kGemvMaxRoutes) return KTMI_MODE_GROUPED;
-  return L && tokens * top_k >= kDecodeMinRoutes && decode_mfma_fits(L, tokens, top_k) ? KTMI_MODE_DECODE
-                                                                                       : KTMI_MODE_GEMV;
+  if (!L || !decode_mfma_fits(L, tokens, top_k)) return KTMI_MODE_GEMV;
+  return tokens * top_k >= kDecodeMinRoutes || !decode_layer_fits(L, tokens, top_k) ? KTMI_MODE_DECODE : KTMI_MODE_GEMV;
 }
 
 static int64_t gemv_layer_workspace(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
@@ -263,10 +265,9 @@ int ktmi_moe_layer(const ktmi_layer* L, const void* x, const float* topk_w, cons
   const int64_t K = L->hidden, N = L->inter;
   if (mode == KTMI_MODE_DECODE) {
     KTMI_REQUIRE(decode_mfma_fits(L, tokens, top_k), KTMI_EINVAL,
-                 "moe_layer: the decode mode takes at most %d routes of %d tokens, at most 512 slots, hidden and "
-                 "intermediate sizes that are multiples of 256, and rows that fit its staging (16 gate and 16 up "
-                 "rows in %d bytes, 16 down rows in %d bytes)",
-                 DM_MAX_ROUTES, DM_MAX_TOKENS, DM_GU_LDS, DM_DOWN_WAVE_LDS);
+                 "moe_layer: the decode mode takes at most %d routes of %d tokens, at most 512 slots, and hidden and "
+                 "intermediate sizes that are multiples of 256",
+                 DM_MAX_ROUTES, DM_MAX_TOKENS);
     return launch_decode_mfma(L, (const uint16_t*)x, topk_w, slot_ids, tokens, top_k, (uint16_t*)y, (uint8_t*)workspace,
                               s);
   }

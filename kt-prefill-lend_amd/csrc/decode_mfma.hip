@@ -1,20 +1,25 @@
-// Decode-sized hot-expert layer on the matrix cores (KTMI_MODE_DECODE): three launches for up
-// to DM_MAX_ROUTES routes and DM_MAX_TOKENS tokens, the weights decoded from their GGUF
-// blocks straight into v_mfma_f32_16x16x32_bf16 operands (bpiece.h: the exact dequantised
-// values, one bf16 rounding, the values the grouped prefill kernels and the dequant entry
-// point use), the routes of one slot as the MFMA's 16 columns.
+// Decode-sized hot-expert layer on the matrix cores (KTMI_MODE_DECODE, and the shortest chunks
+// of KTMI_MODE_GROUPED): three launches, the weights decoded from their GGUF blocks straight
+// into v_mfma_f32_16x16x32_bf16 operands (bpiece.h: the exact dequantised values, one bf16
+// rounding, the values the grouped prefill kernels and the dequant entry point use), the routes
+// of one slot as the MFMA's 16 columns.
 //
-//   dm_gate_up      block (k-th slot with routes, 16 intermediate rows): the block's 16 gate
-//                   and 16 up rows staged in LDS by direct loads; the 4 waves split the
-//                   hidden dimension, each lane decodes its share of the gate row and the up
-//                   row it owns and multiplies them against the bf16 x rows of the slot's
-//                   routes; the partial sums meet in LDS, h = bf16(silu(g) * u) (the grouped
-//                   epilogue's) goes to h [R, N] of the routes.
-//   dm_down         block (k-th slot with routes, 64 hidden rows): each wave stages 16 down
-//                   rows of the slot in LDS by direct loads, runs them against the h rows of
+//   dm_gate_up      block (k-th slot with routes, 16 intermediate rows): the 4 waves split the
+//                   hidden dimension; each moves its columns of the 16 gate and 16 up rows
+//                   through a ring in LDS, decodes them and multiplies them against the bf16 x
+//                   rows of the slot's routes; the partial sums meet in LDS,
+//                   h = bf16(silu(g) * u) (the grouped epilogue's) goes to h [R, N].
+//   dm_down         block (k-th slot with routes, 64 or 128 hidden rows): each wave runs its 16
+//                   or 32 down rows of the slot through a ring of its own against the h rows of
 //                   the slot's routes and writes each route's outputs, rounded to bf16 (the
 //                   reference's per-route bf16 output), to yv [R, K].
 //   dm_combine      the weighted top-k sum in k order (hot/kt_gguf_hot.py:43-71).
+//
+// What bounds them: the touched weights' bytes (up to 5 TB/s on large experts) and, close
+// behind, the decode (2.5 to 4 VALU a value); on small layers the three launches. The weights
+// pass through LDS one super-block column at a time, so any row length runs at the same
+// occupancy: the 7168 x 2048 Q4_K/Q6_K layer with 24 slots at 5 tokens takes 87 us (stage-by-
+// stage GEMV 189-244), the 2048 x 768 Q8_0 layer with 16 slots at 24 tokens 34 us (168-174).
 //
 // Lane map (16x16x32 operands): row or column l % 16, k-chunk g = l / 16 (8 values). Lane
 // group g holds the piece of BPiece step SUB = 2 s + (g & 1), half g >> 1 of each 128-value
@@ -40,15 +45,10 @@ namespace ktmi {
 
 namespace {
 
-constexpr int DM_WAVES = 4;                   // gate/up block: waves over the hidden dimension
+constexpr int DM_WAVES = 4;                   // waves of a block
 constexpr int DM_THREADS = DM_WAVES * 64;
-constexpr int DM_RT = 16;                     // intermediate rows per gate/up block
-constexpr int DN_WAVES = 4;                   // down block: waves over the block's hidden rows
-constexpr int DN_THREADS = DN_WAVES * 64;
-constexpr int DN_ROWS = 16;                   // hidden rows per down wave (the MFMA's rows)
-constexpr int DN_TILE = DN_WAVES * DN_ROWS;   // hidden rows per down block
-constexpr int DN_WREG = DM_DOWN_WAVE_LDS;     // a wave's staged down rows
-static_assert(DM_MAX_ROUTES <= 256, "four routes a lane; a route id fits a byte");
+constexpr int DM_RT = 16;                     // rows of a row tile (the MFMA's rows)
+constexpr int DM_ROUTES = 1024;               // routes of a call these kernels take
 
 __device__ __forceinline__ f32x4_t mfma16(const bf16x8_t& a, const bf16x8_t& b, const f32x4_t& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -69,13 +69,14 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The call's routes, four a lane: route 64 i + lane has slot sid[i] (-1: no slot here).
+// The call's routes, NR a lane: route 64 i + lane has slot sid[i] (-1: no slot here).
+template <int NR>
 struct WaveRoutes {
-  int sid[4];
+  int sid[NR];
   __device__ __forceinline__ void load(const int32_t* __restrict__ slot_ids, int R, int S) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NR; ++i) {
       const int r = 64 * i + lane;
       const int s = r < R ? slot_ids[r] : -1;
       sid[i] = s >= 0 && s < S ? s : -1;
@@ -99,39 +100,38 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
                     __builtin_amdgcn_readlane((int)v, 32) | __builtin_amdgcn_readlane((int)v, 48));
 }
 
-// The slots with routes as 16 words of 32 slots (S <= 512), the same in every lane (scalar
+// The slots with routes as 8 words of 64 slots (S <= 512), the same in every lane (scalar
 // registers): each word is the OR over the wave of the lanes' own route bits.
 struct SlotSet {
-  static constexpr int NW = 16;
-  uint32_t word[NW];
-  int total;
-  __device__ __forceinline__ void build(const WaveRoutes& wr, int S) {
+  static constexpr int NW = 8;
+  uint32_t word[2 * NW];
+  template <int NR>
+  __device__ __forceinline__ void build(const WaveRoutes<NR>& wr, int S) {
     const int nw = (S + 31) >> 5;
-    total = 0;
 #pragma unroll
-    for (int c = 0; c < NW; ++c) {
+    for (int c = 0; c < 2 * NW; ++c) {
       word[c] = 0u;
       if (c < nw) {  // uniform
         uint32_t m = 0u;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          m |= wr.sid[i] >= 0 && (wr.sid[i] >> 5) == c ? 1u << (wr.sid[i] & 31) : 0u;
+        for (int i = 0; i < NR; ++i) m |= (wr.sid[i] >> 5) == c ? 1u << (wr.sid[i] & 31) : 0u;  // -1 >> 5 is -1
         word[c] = wave_or(m);
-        total += __popc(word[c]);
       }
     }
   }
-  // the k-th slot with routes in ascending order, -1 past the last (uniform over the wave)
+  // the k-th slot with routes in ascending order, -1 past the last (uniform over the wave): in
+  // the word that holds it, the lane whose bit is set with k set bits below it
   __device__ __forceinline__ int kth(int k) const {
-    if (k >= total) return -1;
     int e = -1;
 #pragma unroll
     for (int c = 0; c < NW; ++c) {
-      const int n = __popc(word[c]);
-      if (e < 0 && k < n) {  // uniform: the word holding it; its k lowest set bits cleared
-        uint32_t v = word[c];
-        for (int j = k; j > 0; --j) v &= v - 1u;
-        e = 32 * c + __ffs(v) - 1;
+      const uint32_t lo = word[2 * c], hi = word[2 * c + 1];
+      const int n = __popc(lo) + __popc(hi);
+      if (e < 0 && k >= 0 && k < n) {  // uniform
+        const int lane = threadIdx.x & 63;
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+        const uint32_t bit = ((lane < 32 ? lo : hi) >> (lane & 31)) & 1u;
+        e = 64 * c + (int)__builtin_ctzll(__ballot(bit && (int)below == k));
       }
       k -= n;
     }
@@ -139,24 +139,28 @@ struct SlotSet {
   }
 };
 
-// The routes of slot e in ascending order at mem[0 .. m) (LDS private to the wave, a byte a
-// route: route ids are below DM_MAX_ROUTES = 256); returns m. m <= tokens unless a token
-// lists a slot twice; either way every route of the slot is listed.
-__device__ __forceinline__ int slot_routes(const WaveRoutes& wr, int e, uint8_t* mem) {
+// The routes of slot e in ascending order at mem[0 .. m) (LDS; every wave of the block writes
+// the same list and reads what it wrote itself, so the block needs no barrier); returns m.
+// m <= tokens unless a token lists a slot twice; either way every route of the slot is listed.
+template <int NR>
+__device__ __forceinline__ int slot_routes(const WaveRoutes<NR>& wr, int e, uint16_t* mem) {
   const int lane = threadIdx.x & 63;
   const uint64_t below = (1ull << lane) - 1ull;
   int base = 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < NR; ++i) {
     const bool hit = wr.sid[i] == e;
     const uint64_t b = __ballot(hit);
     const int at = base + __popcll(b & below);
-    if (hit) mem[at] = (uint8_t)(64 * i + lane);
+    if (hit) mem[at] = (uint16_t)(64 * i + lane);
     base += __popcll(b);
   }
   wave_fence();
   return base;
 }
+
+// s_waitcnt operand: at most n vector memory operations outstanding (expcnt and lgkmcnt free)
+constexpr int dm_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
 // K offset inside a super-block column of the 8 values lane group (p, h) holds for MFMA j of
 // double step S2 (the piece's values 8j..8j+7)
@@ -166,278 +170,308 @@ __device__ __forceinline__ int kpos(int p, int h, int j) {
   return BP::template ksub_hp<S2>(p) + BP::coff(q);
 }
 
-// One block per (k-th slot with routes, 16 intermediate rows). The block's 16 gate rows and
-// 16 up rows (two contiguous ranges of the slot tensor, 32 row_bytes(K) bytes) are moved into
-// LDS by direct loads all issued at once, so the weights in flight cost no registers and
-// three blocks share a CU; the 4 waves then take a quarter of the hidden dimension each,
-// decode their share of the staged rows into MFMA operands and multiply them with the x rows
-// of the slot's routes (loaded into registers behind the direct loads); the partial sums
-// meet in LDS and h = bf16(silu(g) * u) goes to h [R, N] of the routes.
-template <int TYPE>
-__global__ __launch_bounds__(DM_THREADS) void dm_gate_up(const uint16_t* __restrict__ x, int K, int N,
-                                                         const int32_t* __restrict__ slot_ids, int R, int S,
-                                                         int top_k, const uint8_t* __restrict__ W13, int w_is_table,
-                                                         int64_t w_stride, uint16_t* __restrict__ hbuf) {
+// A wave's weights on their way to the matrix cores: NT tiles of 16 rows, one super-block
+// column (256 values of every row) at a time, moved into the wave's own LDS ring of NB columns
+// by direct loads. A staged row keeps its bytes from the 16-byte boundary below them, CH chunks
+// of 16 bytes a row: an odd number, so the 16 rows of a tile fall into different banks.
+template <int TYPE, int NT, int NB>
+struct ColRing {
+  static constexpr int QB = TYPE == GGML_Q8_0 ? 8 * QB8_0 : (int)Fmt<TYPE>::QB;  // a row's bytes of a column
+  // 16-byte aligned columns (QB and row_bytes multiples of 16) or 2-byte aligned ones
+  static constexpr bool ALIGNED = QB % 16 == 0;
+  static constexpr int USED = (QB + (ALIGNED ? 0 : 14) + 15) / 16;  // chunks that hold the row's bytes
+  static constexpr int CH = USED | 1;
+  static constexpr int ROW = 16 * CH;
+  static constexpr int BUF = NT * DM_RT * ROW;
+  static constexpr int BYTES = NB * BUF;  // a wave's ring
+  static constexpr int NI = (NT * DM_RT * CH + 63) / 64;  // direct loads a column
+  uint8_t* lds;
+  const uint8_t* base;  // the slot's matrix from the 16-byte boundary below it
+  uint32_t bytes;
+  uint32_t off[NI];    // the lane's chunk of load i: its row's offset (+ 16 chunk where ALIGNED)
+  uint32_t roff[NT];   // offset of this lane's own row (lane % 16) of tile t
+  // row0[t]: first row of tile t in the slot's matrix at wexp (rb bytes a row, rows of them)
+  __device__ __forceinline__ void init(uint8_t* region, const uint8_t* wexp, int rows, int64_t rb,
+                                       const int (&row0)[NT]) {
+    const int lane = threadIdx.x & 63;
+    lds = region;
+    const uint32_t mis = (uint32_t)(uintptr_t)wexp & 15u;
+    base = wexp - mis;
+    bytes = (uint32_t)(rows * rb) + mis;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int q = 64 * i + lane, row = q / CH;
+      const int t = min(row / DM_RT, NT - 1);
+      off[i] = mis + (uint32_t)((row0[t] + row % DM_RT) * rb) + (ALIGNED ? 16u * (uint32_t)(q % CH) : 0u);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) roff[t] = mis + (uint32_t)((row0[t] + (lane & 15)) * rb);
+  }
+  // column sb into buffer buf; where more is false the same loads go past the end of a buffer
+  // of no bytes (zeros, no memory access), so that the count of operations in flight does not
+  // depend on the column
+  __device__ __forceinline__ void issue(int sb, int buf, bool more) const {
+    const int lane = threadIdx.x & 63;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, more ? bytes : 0u, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int q = 64 * i + lane;
+      const uint32_t o = ALIGNED ? off[i] : ((off[i] + (uint32_t)(sb * QB)) & ~15u) + 16u * (uint32_t)(q % CH);
+      if ((i < NI - 1 || q < NT * DM_RT * CH) && (USED == CH || q % CH < USED))
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            rsrc, (__attribute__((address_space(3))) void*)(lds + buf * BUF + 1024 * i), 16, (int)o,
+            ALIGNED ? sb * QB : 0, 0, 0);
+    }
+  }
+  // the lane's row of tile t in buffer buf, as a row that starts at column sb
+  __device__ __forceinline__ const uint8_t* row(int sb, int buf, int t) const {
+    return lds + buf * BUF + (16 * t + (threadIdx.x & 15)) * ROW + (ALIGNED ? 0 : (roff[t] + (uint32_t)(sb * QB)) & 15u);
+  }
+};
+
+// Columns [sb0, sb1) of the ring's NT tiles against the activation rows of ng <= G groups of 16
+// routes (a row per lane % 16 and group, at byte xoff[cg] of act; past the routes an offset past
+// the buffer, whose loads return zeros): acc[t][cg] += tile t x group cg.
+//
+// Order of a column's memory operations: the activation loads of its first half (at G = 1 of
+// both halves), its weight bytes out of LDS into registers, the direct loads of column
+// sb + NB into the buffer just read, then (G > 1) the activation loads of the second half; the
+// decode of a half (about 450 VALU cycles a tile) runs while its activation loads are in flight.
+template <int TYPE, int NT, int NB, int G>
+__device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring, const __amdgpu_buffer_rsrc_t& act,
+                                               const uint32_t (&xoff)[G], int ng, int sb0, int sb1,
+                                               const uint32_t* grid, f32x4_t (&acc)[NT][G]) {
   using BP = BPiece<TYPE>;
-  // one LDS object (see the down kernel): staged rows, the waves' partial sums, their
-  // scratch, the IQ3_S codebook
-  constexpr int PART_OFF = DM_GU_LDS;
-  constexpr int SCR_OFF = PART_OFF + DM_WAVES * 2 * 4 * 64 * 4;
-  constexpr int GRID_OFF = SCR_OFF + DM_WAVES * DM_MAX_ROUTES;
-  constexpr int LDS_BYTES = GRID_OFF + (TYPE == GGML_IQ3_S ? 2048 : 16);
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_BYTES];
-  float (*part)[2][4][64] = (float(*)[2][4][64])(smem + PART_OFF);  // [wave][tile: gate, up]
-  uint8_t (*scratch)[DM_MAX_ROUTES] = (uint8_t(*)[DM_MAX_ROUTES])(smem + SCR_OFF);
-  uint32_t* grid = (uint32_t*)(smem + GRID_OFF);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = N / DM_RT;
-  const int kslot = blockIdx.x / G, rg = blockIdx.x - kslot * G;
-  if constexpr (TYPE == GGML_IQ3_S) stage_iq3s_sel(grid);
-  WaveRoutes wr;
+  const int lane = threadIdx.x & 63;
+  const int p = (lane >> 4) & 1, h = (lane >> 5) & 1;
+  bf16x8_t xv[G == 1 ? 2 : 1][G][4];
+  auto xissue = [&](int sb, auto s2c) {
+    constexpr int S2 = decltype(s2c)::value;
+#pragma unroll
+    for (int cg = 0; cg < G; ++cg)
+      if (cg < ng)  // uniform
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          xv[G == 1 ? S2 : 0][cg][j] = __builtin_bit_cast(
+              bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                            act, (int)(xoff[cg] + 2u * (uint32_t)(kpos<BP, S2>(p, h, j))), 512 * sb, 0));
+  };
+  using H0 = std::integral_constant<int, 0>;
+  using H1 = std::integral_constant<int, 1>;
+  int buf = 0;
+  for (int sb = sb0; sb < sb1; ++sb) {
+    xissue(sb, H0{});
+    if constexpr (G == 1) xissue(sb, H1{});
+    __builtin_amdgcn_sched_barrier(0);  // the activation loads stay ahead of the wait that counts them
+    // the column's direct loads have landed once at most the younger operations are in flight:
+    // the next column's (NB = 2) and this column's activation loads (at least 4, 8 at G = 1)
+    constexpr int NX = G == 1 ? 8 : 4;
+    __builtin_amdgcn_s_waitcnt(dm_vmcnt((NB - 1) * ColRing<TYPE, NT, NB>::NI + NX));
+    wave_fence();
+    typename BP::Head hd[NT];
+    typename BP::Raw raw[NT][2];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const uint8_t* row = ring.row(sb, buf, t);
+      BP::template load_head<LMem>(row, 0, h, hd[t]);
+      BP::template load_hp<0, LMem>(row, 0, h, p, grid, raw[t][0]);
+      BP::template load_hp<1, LMem>(row, 0, h, p, grid, raw[t][1]);
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the buffer has been read
+    wave_fence();
+    ring.issue(sb + NB, buf, sb + NB < sb1);
+    auto half = [&](auto s2c) {
+      constexpr int S2 = decltype(s2c)::value;
+      uint32_t a[NT][16];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) BP::template decode_hp<S2>(hd[t], raw[t][S2], grid, p, a[t]);
+#pragma unroll
+      for (int cg = 0; cg < G; ++cg)
+        if (cg < ng)  // uniform
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              acc[t][cg] = mfma16(words8(&a[t][4 * j]), xv[G == 1 ? S2 : 0][cg][j], acc[t][cg]);
+    };
+    half(H0{});
+    if constexpr (G > 1) xissue(sb, H1{});
+    half(H1{});
+    buf = NB == 2 ? buf ^ 1 : 0;
+  }
+  __builtin_amdgcn_s_waitcnt(dm_vmcnt(0));  // the loads past the last column have written their zeros
+}
+
+// The k-th slot with routes of this block, its routes listed in mem: (slot, route count), slot
+// -1 past the slots with routes (the same in every wave)
+template <int NR>
+__device__ __forceinline__ int2 block_slot(const int32_t* __restrict__ slot_ids, int R, int S, int kslot,
+                                           uint16_t* mem) {
+  WaveRoutes<NR> wr;
   wr.load(slot_ids, R, S);
   SlotSet ss;
   ss.build(wr, S);
   const int e = ss.kth(kslot);
-  if (e < 0) return;  // the same in every wave: past the slots with routes
-  // the slot's routes and the first 16 routes' x offsets before the direct loads into LDS
-  uint8_t* mem = scratch[wave];
-  const int m = slot_routes(wr, e, mem);
-  const int ncg = (m + 15) >> 4;  // 16-route column groups
-  const int r = lane & 15, p = (lane >> 4) & 1, h = (lane >> 5) & 1;
+  if (e < 0) return make_int2(-1, 0);
+  return make_int2(e, slot_routes(wr, e, mem));
+}
+
+// waves a SIMD the registers leave room for without spilling
+template <int TYPE, int G>
+constexpr int dm_waves() {
+  return G == 4 ? 2 : G == 1 ? (TYPE == GGML_Q4_K ? 4 : 3) : TYPE == GGML_Q4_K || TYPE == GGML_Q8_0 ? 3 : 2;
+}
+
+// One block per (k-th slot with routes, 16 intermediate rows): each wave takes a quarter of the
+// hidden dimension of the block's 16 gate and 16 up rows, the partial sums meet in LDS and
+// h = bf16(silu(g) * u) goes to h [R, N] of the routes. G groups of 16 routes share a pass over
+// the weights.
+template <int TYPE, int G, int NR, int NB>
+__global__ __launch_bounds__(DM_THREADS, (dm_waves<TYPE, G>())) void dm_gate_up(const uint16_t* __restrict__ x, int K, int N,
+                                                         const int32_t* __restrict__ slot_ids, int R, int S,
+                                                         int top_k, const uint8_t* __restrict__ W13, int w_is_table,
+                                                         int64_t w_stride, uint16_t* __restrict__ hbuf) {
+  using Ring = ColRing<TYPE, 2, NB>;
+  // one LDS object (a second one makes the compiler wait for every direct load before each LDS
+  // read): the IQ3_S codebook, the route list, the waves' rings, over them the partial sums
+  constexpr int GRID = TYPE == GGML_IQ3_S ? 2048 : 0;
+  constexpr int RING_OFF = GRID + NR * 64 * 2;
+  constexpr int PART = DM_WAVES * 2 * G * 4 * 64 * 4;
+  constexpr int RINGS = DM_WAVES * Ring::BYTES;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[RING_OFF + (RINGS > PART ? RINGS : PART)];
+  uint32_t* grid = (uint32_t*)smem;
+  uint16_t* mem = (uint16_t*)(smem + GRID);
+  float (*part)[2][G][4][64] = (float(*)[2][G][4][64])(smem + RING_OFF);  // [wave][tile: gate, up]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int NG = N / DM_RT;
+  const int kslot = blockIdx.x / NG, rg = blockIdx.x - kslot * NG;
+  if constexpr (TYPE == GGML_IQ3_S) stage_iq3s_sel(grid);
+  const int2 em = block_slot<NR>(slot_ids, R, S, kslot, mem);
+  const int e = em.x, m = em.y;
+  if (e < 0) return;
+  if constexpr (TYPE == GGML_IQ3_S) __syncthreads();  // the codebook
+  const int r = lane & 15;
   const uint32_t x_bytes = (uint32_t)(R / top_k) * (uint32_t)K * 2u;
-  uint32_t xoff = r < m ? (uint32_t)(mem[r] / top_k) * (uint32_t)K * 2u : x_bytes;
-  const int64_t rb = row_bytes(K, TYPE);
-  const int range = DM_RT * (int)rb;  // bytes of 16 rows, a multiple of 16
-  {
-    // the gate range at smem, the up range at smem + range: 1 KB pieces over the waves, the
-    // last piece of a range moved back to end at the range's end (its bytes written twice,
-    // with the same values)
-    const uint8_t* wexp = w_is_table ? (const uint8_t*)((const int64_t*)W13)[e] : W13 + (int64_t)e * w_stride;
-    const int npc = (range + 1023) >> 10;
-    for (int q = wave; q < 2 * npc; q += DM_WAVES) {  // uniform per wave
-      const int t = q >= npc, qi = q - t * npc;
-      const int off = min(qi << 10, range - 1024);  // range >= 1024: decode_mfma_fits
-      const uint8_t* src = wexp + ((int64_t)(t ? N : 0) + (int64_t)DM_RT * rg) * rb;
-      const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)src, (short)0, (uint32_t)range, 0x00020000);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (__attribute__((address_space(3))) void*)(smem + t * range + off), 16,
-                                               off + 16 * lane, 0, 0, 0);
-    }
-  }
-  const uint8_t* wrow[2] = {smem + r * (int)rb, smem + range + r * (int)rb};  // staged gate row r, up row r
-  // activation operand: column c = 16 cg + r is the slot's c-th route (its token's x row);
-  // columns past the routes read past the buffer, which returns zeros
   const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, x_bytes, 0x00020000);
-  int kp[2][4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    kp[0][j] = kpos<BP, 0>(p, h, j);
-    kp[1][j] = kpos<BP, 1>(p, h, j);
-  }
-  auto xload = [&](uint32_t off, int sb, int k) {
-    const u32x4_t v = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, off + 2u * (uint32_t)(256 * sb + k), 0, 0));
-    return __builtin_bit_cast(bf16x8_t, v);
-  };
-  // this wave's super-block columns
+  const uint8_t* wexp = w_is_table ? (const uint8_t*)((const int64_t*)W13)[e] : W13 + (int64_t)e * w_stride;
+  Ring ring;
+  ring.init(smem + RING_OFF + wave * Ring::BYTES, wexp, 2 * N, row_bytes(K, TYPE), {DM_RT * rg, N + DM_RT * rg});
   const int nsb = K / 256;
   const int per = (nsb + DM_WAVES - 1) / DM_WAVES;
   const int sb0 = wave * per, sb1 = min(nsb, sb0 + per);
-  f32x4_t acc[2][2];  // [tile: gate, up][two in turn, so back-to-back MFMAs do not wait for each other]
-  // two super-block columns (sb, and sb + 1 when has1) of both tiles: every LDS read of the
-  // four pieces first, then their decodes and MFMAs (one wave a SIMD at small T: the reads'
-  // latency is paid once, not four times)
-  bf16x8_t xa[2][4], xc[2][4];  // the x operands of the two columns
-  auto compute2 = [&](int sb, bool has1) {
-    typename BP::Head hd[2][2];
-    typename BP::Raw raw[2][2][2];
-    const int sbb = has1 ? sb + 1 : sb;
-#pragma unroll
-    for (int c2 = 0; c2 < 2; ++c2)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int sc = c2 ? sbb : sb;
-        BP::template load_head<LMem>(wrow[t], sc, h, hd[c2][t]);
-        BP::template load_hp<0, LMem>(wrow[t], sc, h, p, grid, raw[c2][t][0]);
-        BP::template load_hp<1, LMem>(wrow[t], sc, h, p, grid, raw[c2][t][1]);
-      }
-#pragma unroll
-    for (int c2 = 0; c2 < 2; ++c2) {
-      if (c2 == 1 && !has1) break;  // uniform
-      const bf16x8_t (&xb)[2][4] = c2 ? xc : xa;
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        uint32_t a[16];
-        BP::template decode_hp<0>(hd[c2][t], raw[c2][t][0], grid, p, a);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[t][j & 1] = mfma16(words8(&a[4 * j]), xb[0][j], acc[t][j & 1]);
-        BP::template decode_hp<1>(hd[c2][t], raw[c2][t][1], grid, p, a);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[t][j & 1] = mfma16(words8(&a[4 * j]), xb[1][j], acc[t][j & 1]);
-      }
-    }
-  };
-  // output (row rr, column c): lane 16 (rr / 4) + c of each wave holds it as element rr % 4;
-  // 16 consecutive threads write one route's 16 values of h (32 bytes)
   const int c = threadIdx.x >> 4, rr = threadIdx.x & 15;
   const int ln = 16 * (rr >> 2) + c, i = rr & 3;
-  // one pass per 16 routes of the slot (a second one only past 16 routes)
-  for (int cg = 0; cg < ncg; ++cg) {
-    if (cg > 0) xoff = 16 * cg + r < m ? (uint32_t)(mem[16 * cg + r] / top_k) * (uint32_t)K * 2u : x_bytes;
-    acc[0][0] = acc[0][1] = acc[1][0] = acc[1][1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    // the x operands of two super-block columns in flight (all of a wave's with K = 2048)
-    auto xissue = [&](int sb, bf16x8_t (&xb)[2][4]) {
+  const int ncg = (m + 15) >> 4;
+  for (int cg0 = 0; cg0 < ncg; cg0 += G) {
+    const int ng = min(G, ncg - cg0);
+    uint32_t xoff[G];
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xb[s2][j] = xload(xoff, sb, kp[s2][j]);
-    };
-    if (sb0 < sb1) xissue(sb0, xa);
-    if (sb0 + 1 < sb1) xissue(sb0 + 1, xc);
-    if (cg == 0) {
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the staged rows (and the x operands)
-      __syncthreads();                    // every wave's pieces; the IQ3_S codebook
+    for (int cg = 0; cg < G; ++cg) {
+      const int col = 16 * (cg0 + cg) + r;
+      xoff[cg] = col < m ? (uint32_t)(mem[col] / top_k) * (uint32_t)K * 2u : x_bytes;
     }
-    for (int sb = sb0; sb < sb1; sb += 2) {
-      compute2(sb, sb + 1 < sb1);
-      if (sb + 2 < sb1) xissue(sb + 2, xa);
-      if (sb + 3 < sb1) xissue(sb + 3, xc);
-    }
-    if (cg > 0) __syncthreads();  // the previous pass has read the partial sums
+    if (cg0 > 0) __syncthreads();  // the previous pass has read the partial sums
+    ring.issue(sb0, 0, sb0 < sb1);
+    if (NB == 2) ring.issue(sb0 + 1, 1, sb0 + 1 < sb1);
+    f32x4_t acc[2][G];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int cg = 0; cg < G; ++cg) acc[0][cg] = acc[1][cg] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    window_columns<TYPE, 2, NB, G>(ring, x_rsrc, xoff, ng, sb0, sb1, grid, acc);
+    __syncthreads();  // every wave has read its ring
 #pragma unroll
-      for (int q = 0; q < 4; ++q) part[wave][t][q][lane] = acc[t][0][q] + acc[t][1][q];
+    for (int cg = 0; cg < G; ++cg)
+      if (cg < ng)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) part[wave][t][cg][q][lane] = acc[t][cg][q];
     __syncthreads();
-    const int col = 16 * cg + c;
-    if (col < m) {
-      float g = 0.0f, u = 0.0f;
+    // output (row rr, column c): lane 16 (rr / 4) + c of each wave holds it as element rr % 4;
+    // 16 consecutive threads write one route's 16 values of h (32 bytes)
 #pragma unroll
-      for (int w = 0; w < DM_WAVES; ++w) {
-        g += part[w][0][i][ln];
-        u += part[w][1][i][ln];
+    for (int cg = 0; cg < G; ++cg) {
+      const int col = 16 * (cg0 + cg) + c;
+      if (col < m) {
+        float g = 0.0f, u = 0.0f;
+#pragma unroll
+        for (int w = 0; w < DM_WAVES; ++w) {
+          g += part[w][0][cg][i][ln];
+          u += part[w][1][cg][i][ln];
+        }
+        hbuf[(int64_t)mem[col] * N + DM_RT * rg + rr] = f2bf(dm_silu_mul(g, u));
       }
-      hbuf[(int64_t)mem[col] * N + DM_RT * rg + rr] = f2bf(dm_silu_mul(g, u));
     }
   }
 }
 
-// One block per (k-th slot with routes, DN_TILE hidden rows); wave w takes the tile's rows
-// 16 w .. 16 w + 15. A wave moves its 16 down rows of the slot (contiguous in the slot
-// tensor) into its LDS region by direct loads, brings the h rows of the slot's routes into
-// registers behind them (L2 hits: every block of the slot reads the same rows), decodes the
-// rows into MFMA operands and writes each route's 16 outputs, rounded to bf16 (the
-// reference's per-route bf16 output), to yv [R, K]. The weighted top-k sum is a launch of its
-// own (dm_combine): inside this one, the blocks of a tile would have to order themselves
-// through device-scope fences, which write back and invalidate the whole L2 of their XCD.
-template <int TYPE>
-__global__ __launch_bounds__(DN_THREADS) void dm_down(const uint16_t* __restrict__ hbuf, int K, int N,
+// One block per (k-th slot with routes, 64 NT hidden rows); wave w takes the tile's rows
+// 16 NT w .. over the whole intermediate dimension against the h rows of the slot's routes (L2
+// hits: every block of the slot reads the same rows) and writes each route's outputs, rounded
+// to bf16 (the reference's per-route bf16 output), to yv [R, K]. The weighted top-k sum is a
+// launch of its own (dm_combine): inside this one, the blocks of a tile would have to order
+// themselves through device-scope fences, which write back and invalidate the whole L2 of
+// their XCD.
+template <int TYPE, int NT, int G, int NR, int NB>
+__global__ __launch_bounds__(DM_THREADS, (G == 1 ? 4 : G == 2 ? 3 : 2)) void dm_down(const uint16_t* __restrict__ hbuf, int K, int N,
                                                       const int32_t* __restrict__ slot_ids, int R, int S,
                                                       const uint8_t* __restrict__ W2, int w_is_table, int64_t w_stride,
                                                       uint16_t* __restrict__ yv) {
-  using BP = BPiece<TYPE>;
-  // one LDS object: per wave its staged rows, then the waves' route lists, the IQ3_S codebook
-  constexpr int MEM_OFF = DN_WAVES * DN_WREG;
-  constexpr int GRID_OFF = MEM_OFF + DN_WAVES * DM_MAX_ROUTES;
-  constexpr int LDS_BYTES = GRID_OFF + (TYPE == GGML_IQ3_S ? 2048 : 16);
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[LDS_BYTES];
-  uint32_t* grid = (uint32_t*)(smem + GRID_OFF);
+  using Ring = ColRing<TYPE, NT, NB>;
+  constexpr int GRID = TYPE == GGML_IQ3_S ? 2048 : 0;
+  constexpr int RING_OFF = GRID + NR * 64 * 2;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[RING_OFF + DM_WAVES * Ring::BYTES];
+  uint32_t* grid = (uint32_t*)smem;
+  uint16_t* mem = (uint16_t*)(smem + GRID);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ntile = K / DN_TILE;
+  constexpr int TILE = DM_WAVES * NT * DM_RT;
+  const int ntile = K / TILE;
   const int kslot = blockIdx.x / ntile, tile = blockIdx.x - kslot * ntile;
-  const int c0 = tile * DN_TILE;
   if constexpr (TYPE == GGML_IQ3_S) stage_iq3s_sel(grid);
-  WaveRoutes wr;
-  wr.load(slot_ids, R, S);
-  SlotSet ss;
-  ss.build(wr, S);
-  const int e = ss.kth(kslot);
-  if (e < 0) return;  // the same in every wave: past the slots with routes
-  // the slot's routes and the first column group's h offsets before any direct load into
-  // LDS: the compiler makes an LDS access after such loads wait for them
-  uint8_t* mem = smem + MEM_OFF + DM_MAX_ROUTES * wave;
-  const int m = slot_routes(wr, e, mem);
-  const int ncg = (m + 15) >> 4;
-  const int r = lane & 15, p = (lane >> 4) & 1, h = (lane >> 5) & 1;
+  const int2 em = block_slot<NR>(slot_ids, R, S, kslot, mem);
+  const int e = em.x, m = em.y;
+  if (e < 0) return;
+  if constexpr (TYPE == GGML_IQ3_S) __syncthreads();  // the codebook
+  const int r = lane & 15;
   const uint32_t hrow = 2u * (uint32_t)N;
   const uint32_t h_bytes = (uint32_t)R * hrow;
-  // column c = 16 cg + r of the operand is the slot's c-th route; past the routes the
-  // offset lies past the buffer, whose loads return zeros
-  uint32_t hoff = r < m ? (uint32_t)mem[r] * hrow : h_bytes;
-  const int64_t rb = row_bytes(N, TYPE);
-  const int wbytes = DN_ROWS * (int)rb;  // a multiple of 16, at most DN_WREG (decode_mfma_fits)
-  const int rw0 = c0 + DN_ROWS * wave;
-  uint8_t* const region = smem + wave * DN_WREG;
-  {
-    const uint8_t* wexp = w_is_table ? (const uint8_t*)((const int64_t*)W2)[e] : W2 + (int64_t)e * w_stride;
-    const __amdgpu_buffer_rsrc_t w_rsrc =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(wexp + (int64_t)rw0 * rb), (short)0, (uint32_t)wbytes, 0x00020000);
-    // 1 KB a wave instruction; the lanes past the end of the last piece stay idle
-    for (int q0 = 0; q0 < wbytes; q0 += 1024)
-      if (q0 + 16 * lane < wbytes)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (__attribute__((address_space(3))) void*)(region + q0), 16,
-                                                 q0 + 16 * lane, 0, 0, 0);
-  }
-  const uint8_t* wrow = region + r * (int)rb;
   const __amdgpu_buffer_rsrc_t h_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)hbuf, (short)0, h_bytes, 0x00020000);
-  int kp[2][4];
+  const uint8_t* wexp = w_is_table ? (const uint8_t*)((const int64_t*)W2)[e] : W2 + (int64_t)e * w_stride;
+  const int rw0 = tile * TILE + wave * NT * DM_RT;
+  int row0[NT];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    kp[0][j] = kpos<BP, 0>(p, h, j);
-    kp[1][j] = kpos<BP, 1>(p, h, j);
-  }
-  auto hload = [&](uint32_t off, int sb, int k) {
-    const u32x4_t v = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(h_rsrc, off + 2u * (uint32_t)(256 * sb + k), 0, 0));
-    return __builtin_bit_cast(bf16x8_t, v);
-  };
+  for (int t = 0; t < NT; ++t) row0[t] = rw0 + DM_RT * t;
+  Ring ring;
+  ring.init(smem + RING_OFF + wave * Ring::BYTES, wexp, K, row_bytes(N, TYPE), row0);
   const int nsb = N / 256;
-  f32x4_t acc[2];
-  // one super-block column against the operands hb[S2][j]; two accumulators in turn, so
-  // back-to-back MFMAs do not wait for each other
-  auto compute = [&](int sb, const bf16x8_t (&hb)[2][4]) {
-    typename BP::Head hd;
-    typename BP::Raw raw[2];
-    BP::template load_head<LMem>(wrow, sb, h, hd);
-    BP::template load_hp<0, LMem>(wrow, sb, h, p, grid, raw[0]);
-    BP::template load_hp<1, LMem>(wrow, sb, h, p, grid, raw[1]);
-    uint32_t a[16];
-    BP::template decode_hp<0>(hd, raw[0], grid, p, a);
+  const int ncg = (m + 15) >> 4;
+  for (int cg0 = 0; cg0 < ncg; cg0 += G) {
+    const int ng = min(G, ncg - cg0);
+    uint32_t hoff[G];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j & 1] = mfma16(words8(&a[4 * j]), hb[0][j], acc[j & 1]);
-    BP::template decode_hp<1>(hd, raw[1], grid, p, a);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j & 1] = mfma16(words8(&a[4 * j]), hb[1][j], acc[j & 1]);
-  };
-  for (int cg = 0; cg < ncg; ++cg) {
-    if (cg > 0) hoff = 16 * cg + r < m ? (uint32_t)mem[16 * cg + r] * hrow : h_bytes;
-    acc[0] = acc[1] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    bf16x8_t ha[2][4], hc[2][4];  // two super-block columns in flight
-    auto hissue = [&](int sb, bf16x8_t (&hb)[2][4]) {
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) hb[s2][j] = hload(hoff, sb, kp[s2][j]);
-    };
-    hissue(0, ha);
-    if (nsb > 1) hissue(1, hc);
-    if (cg == 0) {
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the staged rows (and the h operands)
-      wave_fence();
-      if constexpr (TYPE == GGML_IQ3_S) __syncthreads();  // the codebook
+    for (int cg = 0; cg < G; ++cg) {
+      const int col = 16 * (cg0 + cg) + r;
+      hoff[cg] = col < m ? (uint32_t)mem[col] * hrow : h_bytes;
     }
-    for (int sb = 0; sb < nsb; sb += 2) {
-      compute(sb, ha);
-      if (sb + 2 < nsb) hissue(sb + 2, ha);
-      if (sb + 1 < nsb) {
-        compute(sb + 1, hc);
-        if (sb + 3 < nsb) hissue(sb + 3, hc);
-      }
-    }
+    ring.issue(0, 0, true);
+    if (NB == 2) ring.issue(1, 1, nsb > 1);
+    f32x4_t acc[NT][G];
+#pragma unroll
+    for (int cg = 0; cg < G; ++cg)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t][cg] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    window_columns<TYPE, NT, NB, G>(ring, h_rsrc, hoff, ng, 0, nsb, grid, acc);
     // lane l holds rows 4 (l / 16) + i of column l % 16: four consecutive bf16 of yv
-    const int col = 16 * cg + r;
-    if (col < m) {
-      const int rt = mem[col];
-      const uint32_t lo = (uint32_t)f2bf(acc[0][0] + acc[1][0]) | ((uint32_t)f2bf(acc[0][1] + acc[1][1]) << 16);
-      const uint32_t hi = (uint32_t)f2bf(acc[0][2] + acc[1][2]) | ((uint32_t)f2bf(acc[0][3] + acc[1][3]) << 16);
-      *(uint2*)(yv + (int64_t)rt * K + rw0 + 4 * (lane >> 4)) = make_uint2(lo, hi);
+#pragma unroll
+    for (int cg = 0; cg < G; ++cg) {
+      const int col = 16 * (cg0 + cg) + r;
+      if (col < m) {
+        const int rt = mem[col];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const f32x4_t& v = acc[t][cg];
+          *(uint2*)(yv + (int64_t)rt * K + row0[t] + 4 * (lane >> 4)) = make_uint2(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]));
+        }
+      }
     }
   }
 }
@@ -481,6 +515,8 @@ __global__ __launch_bounds__(256) void dm_combine(const uint16_t* __restrict__ y
   *(uint4*)(y + (int64_t)t * K + c) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
+// G (groups of 16 routes that share a pass over the weights) by the tokens, the routes a slot has unless
+// a token lists it twice; NR (ids a lane of the membership) by the routes
 template <int TYPE>
 int launch_dm_gate_up(const ktmi_layer* L, const uint16_t* x, const int32_t* slot_ids, int64_t tokens, int64_t top_k,
                       uint16_t* hbuf, hipStream_t stream) {
@@ -489,8 +525,15 @@ int launch_dm_gate_up(const ktmi_layer* L, const uint16_t* x, const int32_t* slo
   // blocks numbered (k-th slot with routes, row group), row group fastest; the blocks past
   // the slots with routes exit at once
   const unsigned nb = (unsigned)(S < R ? S : R) * (unsigned)(N / DM_RT);
-  dm_gate_up<TYPE><<<nb, DM_THREADS, 0, stream>>>(x, (int)K, (int)N, slot_ids, (int)R, (int)S, (int)top_k,
-                                                  (const uint8_t*)L->w13, L->w_is_table, st13, hbuf);
+#define KTMI_GU(G, NR)                                                                                        \
+  dm_gate_up<TYPE, G, NR, 2><<<nb, DM_THREADS, 0, stream>>>(x, (int)K, (int)N, slot_ids, (int)R, (int)S, (int)top_k, \
+                                                            (const uint8_t*)L->w13, L->w_is_table, st13, hbuf)
+  if (R <= 256) {
+    if (tokens <= 16) KTMI_GU(1, 4); else if (tokens <= 32) KTMI_GU(2, 4); else KTMI_GU(4, 4);
+  } else {
+    if (tokens <= 32) KTMI_GU(2, 16); else KTMI_GU(4, 16);
+  }
+#undef KTMI_GU
   KTMI_HIP_TRY(hipGetLastError());
   return KTMI_OK;
 }
@@ -502,9 +545,15 @@ int launch_dm_down(const ktmi_layer* L, const uint16_t* hbuf, const int32_t* slo
   const int64_t st2 = K * row_bytes(N, TYPE);
   // blocks numbered (k-th slot with routes, hidden tile), tile fastest; the blocks past the
   // slots with routes exit at once
-  const unsigned nb = (unsigned)(S < R ? S : R) * (unsigned)(K / DN_TILE);
-  dm_down<TYPE><<<nb, DN_THREADS, 0, stream>>>(hbuf, (int)K, (int)N, slot_ids, (int)R, (int)S, (const uint8_t*)L->w2,
-                                               L->w_is_table, st2, yv);
+#define KTMI_DN(NT, G, NR)                                                                                     \
+  dm_down<TYPE, NT, G, NR, 2><<<(unsigned)(S < R ? S : R) * (unsigned)(K / (64 * NT)), DM_THREADS, 0, stream>>>( \
+      hbuf, (int)K, (int)N, slot_ids, (int)R, (int)S, (const uint8_t*)L->w2, L->w_is_table, st2, yv)
+  if (R <= 256) {
+    if (tokens <= 16) KTMI_DN(1, 1, 4); else if (tokens <= 32) KTMI_DN(1, 2, 4); else KTMI_DN(1, 4, 4);
+  } else {
+    if (tokens <= 32) KTMI_DN(2, 2, 16); else KTMI_DN(2, 4, 16);
+  }
+#undef KTMI_DN
   KTMI_HIP_TRY(hipGetLastError());
   const unsigned nc = (unsigned)((tokens * (K / 8) + 255) / 256);
   dm_combine<<<nc, 256, 0, stream>>>(yv, slot_ids, topk_w, (int)tokens, (int)top_k, (int)S, (int)K, y);
@@ -514,12 +563,22 @@ int launch_dm_down(const ktmi_layer* L, const uint16_t* hbuf, const int32_t* slo
 
 }  // namespace
 
+// what the kernels take, whatever the mode
+static bool window_shape(const ktmi_layer* L) {
+  return L->hidden % 256 == 0 && L->inter % 256 == 0 && L->n_slots <= 512;
+}
+
 bool decode_mfma_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
-  if (L->hidden % 256 || L->inter % 256) return false;
-  const int64_t range13 = DM_RT * row_bytes(L->hidden, L->type13);  // 16 gate (or up) rows
-  const int64_t rows2 = DN_ROWS * row_bytes(L->inter, L->type2);    // a down wave's 16 rows
-  return tokens * top_k <= DM_MAX_ROUTES && tokens <= DM_MAX_TOKENS && L->n_slots <= 512 &&
-         L->hidden % DN_TILE == 0 && range13 >= 1024 && 2 * range13 <= DM_GU_LDS && rows2 <= DN_WREG;
+  return window_shape(L) && tokens * top_k <= DM_MAX_ROUTES && tokens <= DM_MAX_TOKENS;
+}
+
+// The chunks the grouped mode gives to these kernels: at 40 tokens they take 42 / 53 / 58 / 148 us
+// (2048 x 768 Q8_0 with 16 slots, 2048 x 512 Q4_K/Q6_K with 40, 2048 x 512 IQ3_S with 48,
+// 7168 x 2048 Q4_K with 16) against the grouped GEMMs' 61 / 67 / 78 / 192; at 77 tokens 54 / 61 /
+// 78 against 60 / 67 / 80, at 128 tokens they are slower on every one: a slot's x and h rows,
+// one 16-byte piece a lane from 16 rows at a time, are then what their loads are busy with.
+bool window_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
+  return window_shape(L) && tokens * top_k <= DM_ROUTES && tokens <= 64;
 }
 
 namespace {
@@ -534,9 +593,12 @@ int64_t decode_mfma_workspace(const ktmi_layer* L, int64_t tokens, int64_t top_k
 
 int launch_decode_mfma(const ktmi_layer* L, const uint16_t* x, const float* topk_w, const int32_t* slot_ids,
                        int64_t tokens, int64_t top_k, uint16_t* y, uint8_t* ws, hipStream_t stream) {
-  const int64_t R = tokens * top_k;
-  uint16_t* hbuf = (uint16_t*)ws;
-  uint16_t* yv = (uint16_t*)(ws + up256(R * L->inter * 2));
+  return launch_window(L, x, topk_w, slot_ids, tokens, top_k, y, (uint16_t*)ws,
+                       (uint16_t*)(ws + up256(tokens * top_k * L->inter * 2)), stream);
+}
+
+int launch_window(const ktmi_layer* L, const uint16_t* x, const float* topk_w, const int32_t* slot_ids, int64_t tokens,
+                  int64_t top_k, uint16_t* y, uint16_t* hbuf, uint16_t* yv, hipStream_t stream) {
   record_stage(0, stream);
   record_stage(1, stream);
   int rc;

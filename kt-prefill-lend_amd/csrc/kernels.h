@@ -36,13 +36,15 @@ int64_t decode_layer_workspace(const ktmi_layer* L, int64_t tokens, int64_t top_
 int launch_decode_layer(const ktmi_layer* L, const uint16_t* x, const float* topk_w, const int32_t* slot_ids,
                         int64_t tokens, int64_t top_k, uint16_t* y, uint8_t* ws, hipStream_t stream);
 
-// Decode-sized layer on the matrix cores (decode_mfma.hip): two launches for up to
-// DM_MAX_ROUTES routes of at most DM_MAX_TOKENS tokens; a down wave stages 16 rows of a slot
-// in an LDS region of DM_DOWN_WAVE_LDS bytes.
+// Decode-sized layer on the matrix cores (decode_mfma.hip): three launches. The decode mode
+// takes up to DM_MAX_ROUTES routes of at most DM_MAX_TOKENS tokens; the grouped mode runs the
+// same kernels on its shortest chunks (window_fits), with h [R, inter] and yv [R, hidden] in
+// its own workspace.
 constexpr int DM_MAX_ROUTES = 256;
 constexpr int DM_MAX_TOKENS = 64;
-constexpr int DM_DOWN_WAVE_LDS = 10 * 1024;
-constexpr int DM_GU_LDS = 40 * 1024;  // gate/up: the block's 16 gate and 16 up rows
+bool window_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k);
+int launch_window(const ktmi_layer* L, const uint16_t* x, const float* topk_w, const int32_t* slot_ids, int64_t tokens,
+                  int64_t top_k, uint16_t* y, uint16_t* hbuf, uint16_t* yv, hipStream_t stream);
 bool decode_mfma_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k);
 int64_t decode_mfma_workspace(const ktmi_layer* L, int64_t tokens, int64_t top_k);
 int launch_decode_mfma(const ktmi_layer* L, const uint16_t* x, const float* topk_w, const int32_t* slot_ids,

@@ -1057,6 +1057,9 @@ int launch_grouped_layer(const ktmi_layer* L, const uint16_t* x, const float* to
   KTMI_REQUIRE(tokens * K * 2 <= 0xFFFF0000ll && R * N * 2 <= 0xFFFF0000ll && R * K * 2 <= 0xFFFF0000ll, KTMI_EINVAL,
                "grouped layer: a pass of %lld tokens exceeds the 32-bit buffer range", (long long)tokens);
   if (tokens == 0) return KTMI_OK;
+  if (window_fits(L, tokens, top_k))
+    return launch_window(L, x, topk_w, slot_ids, tokens, top_k, y, (uint16_t*)(ws + P.off_h), (uint16_t*)(ws + P.off_y),
+                         stream);
   int32_t* hist = (int32_t*)(ws + P.off_counts);
   int32_t* seg = (int32_t*)(ws + P.off_seg);
   int32_t* tseg = (int32_t*)(ws + P.off_tseg);

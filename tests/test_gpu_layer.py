@@ -457,3 +457,33 @@ def test_slot_address_table_matches_contiguous_slots(dev, mode, T):
     got = H.moe_layer(H.layer_desc(t13, t2, w.hidden, w.inter, w.types[0], w.types[2], table=True), x, twd, sd, m)
     torch.cuda.synchronize()
     assert np.array_equal(bf16_bits_of(got), bf16_bits_of(ref))
+
+
+@pytest.mark.parametrize("types", [(R.GGML_Q4_K, R.GGML_Q6_K), (R.GGML_Q6_K, R.GGML_Q4_K), (R.GGML_Q8_0, R.GGML_Q8_0),
+                                   (R.GGML_IQ3_S, R.GGML_IQ3_S)])
+@pytest.mark.parametrize("hidden,inter,T,mode", [(768, 256, 1, "decode"), (1280, 768, 16, "decode"), (256, 512, 17, "decode"),
+                                                 (1280, 256, 32, "grouped"), (512, 1280, 64, "grouped")])
+def test_window_columns(dev, types, hidden, inter, T, mode):
+    """The decode-sized kernels where the split over super-block columns is ragged (1, 3 and 5
+    columns over 4 waves, rings of one column and of more), at 1, 2 and 4 groups of 16 routes a
+    pass, past 256 routes and with a slot listed twice (72 routes of one slot: a second pass);
+    against the fp64 FFN."""
+    L, H, S = _pkg()
+    top_k = 9 if mode == "grouped" else 5
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=hidden, inter=inter, hot=70, experts=128, top_k=top_k, types=(types[0], types[0], types[1]))
+    rng = np.random.default_rng(hidden + inter + T)
+    slot = rng.integers(0, 100, size=(T, top_k)).astype(np.int32)
+    slot = np.where(slot < w.hot, slot, -1).astype(np.int32)
+    slot[:, 0] = 69                 # every token on the last slot
+    slot[: T // 8, 1] = 69          # some twice
+    if T > 40:
+        slot[40:] = np.where(slot[40:] == 69, slot[40:], -1)
+    tw = rng.random((T, top_k)).astype(np.float32)
+    tw /= tw.sum(axis=1, keepdims=True)
+    xb = S.activations(w, T)
+    w13, w2 = S.slot_tensors(w)
+    got = R.bf16_to_f32(_run(dev, w, xb, tw, slot, w13, w2, L.MODE_DECODE if mode == "decode" else L.MODE_GROUPED))
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    l2, l1, cos = R.rel_errors(got, R.ffn_reference(xb, slot, tw, g, d))
+    assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
