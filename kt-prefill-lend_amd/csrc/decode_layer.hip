@@ -212,8 +212,8 @@ __device__ __forceinline__ int lanes_below(uint64_t bal) {
   return __popcll(bal & ((1ull << (threadIdx.x & 63)) - 1));
 }
 
-// lanes per row of the down block: 8, or 16 for rows of 16 units (each lane one unit)
-__host__ __device__ constexpr int dec_lpr(int units) { return units >= 16 ? 16 : 8; }
+// lanes per row of the down block, each lane one unit: 8, or 16 for rows of more than 8 units
+__host__ __device__ constexpr int dec_lpr(int units) { return units > 8 ? 16 : 8; }
 
 // The block's slot and its routes: blocks are numbered k * G + g over the slots that have
 // routes (ascending), so block kslot serves the kslot-th of them. Leaves the slot's routes in

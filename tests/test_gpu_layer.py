@@ -487,3 +487,21 @@ def test_window_columns(dev, types, hidden, inter, T, mode):
     g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
     l2, l1, cos = R.rel_errors(got, R.ffn_reference(xb, slot, tw, g, d))
     assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
+
+
+@pytest.mark.parametrize("types,inter", [((R.GGML_Q4_K, R.GGML_Q4_K), 768), ((R.GGML_Q4_K, R.GGML_Q6_K), 768),
+                                         ((R.GGML_Q8_0, R.GGML_Q8_0), 288), ((R.GGML_Q8_0, R.GGML_Q8_0), 512),
+                                         ((R.GGML_IQ3_S, R.GGML_IQ3_S), 256)])
+def test_fused_decode_down_units(dev, types, inter):
+    """The fused decode launches where a down row has 8, 9, 12 and 16 weight units: every unit
+    is summed (8 lanes a row up to 8 units, 16 past them)."""
+    L, _, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=512, inter=inter, hot=8, experts=32, types=(types[0], types[0], types[1]))
+    _, tw, slot, _ = S.routing(w, 3)
+    xb = S.activations(w, 3)
+    w13, w2 = S.slot_tensors(w)
+    got = R.bf16_to_f32(_run(dev, w, xb, tw, slot, w13, w2, L.MODE_GEMV))
+    exp = R.bf16_to_f32(gemv_layer_oracle(xb, tw, slot, w13, w2, w.types, w.hidden, w.inter))
+    l2, _, _ = R.rel_errors(got, exp)
+    assert l2 < 4e-3, l2
