@@ -24,15 +24,19 @@
 //   Q8_0, IQ3_S: positions [32h, 32h+32) (one Q8_0 block, one IQ3_S 32-group)
 // `off0`/`off1` give the step positions of out[0..7] and out[8..15] (16 values each).
 //
+// A zero value's sign is a plain product's only with decode_hp<S2, SZ = true> (the dequant
+// entry point, whose bytes are its result: d * -0 and the like); elsewhere it may differ, which
+// no sum of products sees.
+//
 // Every SUB-dependent member also exists with the step parity as a run-time value: the
 // `_hp<S2>(..., p)` forms take SUB = 2 S2 + p with S2 a compile-time constant and p a
 // per-lane value (the decode-sized layer's 16x16x32 MFMA operands hold pieces of both
 // parities in one wave); the `<SUB>` forms are those with p constant. One body per format
 // serves both, so the values are the same.
 //
-// 2-byte aligned blocks (Q8_0 34 B, Q6_K 210 B, IQ3_S 110 B) are read with dword loads
-// from the dword-aligned address below and realigned with v_alignbyte; every dword read
-// holds at least one byte of the block, so no load leaves the tensor's pages.
+// The fields of 2-byte aligned blocks are read from global memory where they lie (Q6_K 210 B,
+// IQ3_S 110 B: the hardware takes unaligned addresses), from LDS with dword reads of the
+// dword-aligned address below and v_alignbyte (words()); Q8_0's 34 B see its Raw.
 #pragma once
 #include "formats.h"
 
@@ -69,11 +73,45 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t b) {
   return r;
 }
 
+// d * q + c in one rounding, q the fp16 number in the low (HI = 0) or high half of w: one
+// v_fma_mix_f32. A code of up to 10 bits left as it is in a half-word is the fp16 denormal
+// code * 2^-24, so with d scaled by 2^24 (exact) this is the fp32 FMA of the code itself, and
+// no conversion instruction is needed. With a v_cvt a value the grouped K loop held 890 / 842 /
+// 1088 VALU a super-block column (Q4_K / Q8_0 / Q6_K, the last two with run-time realignment),
+// so 710 / 690 / 812; a 128-route block of one wave a SIMD spends half of its time issuing them
+// (2048 x 512 Q4_K/Q6_K layer, 77 tokens: 67 -> 63.5 us; 7168 x 2048, 300 tokens: 340 -> 322).
+constexpr float kCodeScale = 16777216.0f;  // 2^24
+template <int HI>
+__device__ __forceinline__ float fma_code(float d, uint32_t w, float c) {
+  const _Float16 q = __builtin_bit_cast(_Float16, (uint16_t)(HI ? w >> 16 : w & 0xFFFFu));
+  return __builtin_fmaf(d, (float)q, c);
+}
+// the bf16 pairs of four codes: bytes 0 and 2 of a word as the halves of e, bytes 1 and 3 of o
+__device__ __forceinline__ void codes4(float d, float c, uint32_t e, uint32_t o, uint32_t* out) {
+  out[0] = f2bf2(fma_code<0>(d, e, c), fma_code<0>(d, o, c));
+  out[1] = f2bf2(fma_code<1>(d, e, c), fma_code<1>(d, o, c));
+}
+
 // Where a piece's bytes are read from: global memory (through the caches) or LDS (rows a
-// kernel has staged there, at the same offsets as in the row).
+// kernel has staged there, at the same offsets as in the row). words<N>: N = 1, 2 or 4 dwords
+// from a 2-byte aligned address.
 struct GMem {
   template <typename T>
   __device__ __forceinline__ static T ld(const void* p) { return gload<T>(p); }
+  template <int N>
+  __device__ __forceinline__ static void words(const uint8_t* p, uint32_t* w) {
+    if constexpr (N == 4) {
+      const u32x4_a2_t v = gload<u32x4_a2_t>(p);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = v[i];
+    } else if constexpr (N == 2) {
+      const u32x2_a2_t v = gload<u32x2_a2_t>(p);
+      w[0] = v[0];
+      w[1] = v[1];
+    } else {
+      w[0] = gload<u32_a2_t>(p);
+    }
+  }
 };
 struct LMem {
   // the LDS offset is the generic address's low 32 bits (an address-space cast of a generic
@@ -81,6 +119,28 @@ struct LMem {
   template <typename T>
   __device__ __forceinline__ static T ld(const void* p) {
     return *(const __attribute__((address_space(3))) T*)(uintptr_t)(uint32_t)(uintptr_t)p;
+  }
+  // the last dword read holds the field's last bytes, or (p dword aligned) the two after it:
+  // a staged row is followed by the next one, or by the rest of its own 16-byte chunk
+  template <int N>
+  __device__ __forceinline__ static void words(const uint8_t* p, uint32_t* w) {
+    const uint32_t* a = dword_floor(p);
+    const uint32_t s = byte_shift(p);
+    uint32_t v[N + 1];
+    if constexpr (N == 4) {
+      const u32x4_t q = ld<u32x4_a4_t>(a);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = q[i];
+    } else if constexpr (N == 2) {
+      const u32x2_t q = ld<u32x2_a4_t>(a);
+      v[0] = q[0];
+      v[1] = q[1];
+    } else {
+      v[0] = ld<uint32_t>(a);
+    }
+    v[N] = ld<uint32_t>(a + N);
+#pragma unroll
+    for (int i = 0; i < N; ++i) w[i] = alignbyte(v[i + 1], v[i], s);
   }
 };
 
@@ -141,7 +201,7 @@ struct BPiece<GGML_Q4_K> : NoLookup<BPiece<GGML_Q4_K>> {
   __device__ __forceinline__ static void load_hp(const uint8_t* row, int sb, int h, int p, const uint32_t*, Raw& r) {
     r.q = M::template ld<u32x4_t>(row + sb * QB4_K + 16 + 64 * S2 + 32 * p + 16 * h);
   }
-  template <int S2>
+  template <int S2, bool SZ = false>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t*, int p,
                                                    uint32_t out[16]) {
     const float d = half_bits_to_float(hd.hdr[0] & 0xFFFF);
@@ -156,17 +216,16 @@ struct BPiece<GGML_Q4_K> : NoLookup<BPiece<GGML_Q4_K>> {
     const int sc1 = hi ? (int)(((lo >> 8) & 15) | (((ws >> 14) & 3) << 4)) : (int)((ws >> 8) & 63);
     const int m0 = hi ? (int)(((lo >> 4) & 15) | (((wm >> 6) & 3) << 4)) : (int)(wm & 63);
     const int m1 = hi ? (int)(((lo >> 12) & 15) | (((wm >> 14) & 3) << 4)) : (int)((wm >> 8) & 63);
-    const float d1a = d * (float)sc0, m1a = dmin * (float)m0;
-    const float d1b = d * (float)sc1, m1b = dmin * (float)m1;
-    // 4 bytes = 4 low nibbles (positions off0..) and 4 high nibbles (off1..); each nibble
-    // masked into its own byte converts with one v_cvt_f32_ubyteN
+    // nibbles left in place: low ones (positions off0..) at bit 0 of a half-word, high ones
+    // (off1..) at bit 4, the code times 16
+    const float dn = d * kCodeScale;
+    const float d1a = dn * (float)sc0, m1a = dmin * (float)m0;
+    const float d1b = 0.0625f * (dn * (float)sc1), m1b = dmin * (float)m1;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t nl = and_opaque(r.q[i], 0x0F0F0F0Fu), nh = and_opaque(r.q[i] >> 4, 0x0F0F0F0Fu);
-      out[2 * i] = f2bf2(__builtin_fmaf(d1a, (float)(nl & 0xFF), -m1a), __builtin_fmaf(d1a, (float)((nl >> 8) & 0xFF), -m1a));
-      out[2 * i + 1] = f2bf2(__builtin_fmaf(d1a, (float)((nl >> 16) & 0xFF), -m1a), __builtin_fmaf(d1a, (float)(nl >> 24), -m1a));
-      out[8 + 2 * i] = f2bf2(__builtin_fmaf(d1b, (float)(nh & 0xFF), -m1b), __builtin_fmaf(d1b, (float)((nh >> 8) & 0xFF), -m1b));
-      out[8 + 2 * i + 1] = f2bf2(__builtin_fmaf(d1b, (float)((nh >> 16) & 0xFF), -m1b), __builtin_fmaf(d1b, (float)(nh >> 24), -m1b));
+      const uint32_t w = r.q[i], v = w >> 8;
+      codes4(d1a, -m1a, and_opaque(w, 0x000F000Fu), and_opaque(v, 0x000F000Fu), out + 2 * i);
+      codes4(d1b, -m1b, and_opaque(w, 0x00F000F0u), and_opaque(v, 0x00F000F0u), out + 8 + 2 * i);
     }
   }
   __device__ static int off0(int h) { return 16 * h; }
@@ -179,6 +238,9 @@ struct BPiece<GGML_Q8_0> : NoLookup<BPiece<GGML_Q8_0>> {
   static constexpr int NLOAD2 = 6;  // VMEM instructions of load_next over two consecutive steps
   static constexpr int VPM = 4;    // VALU instructions the GEMM schedule places after each MFMA
   struct Head {};
+  // the 9 dwords from the dword at or below the block, s = byte shift (0 or 2). Read dword
+  // aligned: two unaligned 16-byte loads cost the address unit more than the ninth dword does
+  // (2048 x 768 layer, 512 tokens: 87 against 70 us)
   struct Raw { uint32_t w[9]; uint32_t s; };
   template <int SUB>
   __device__ static int ksub() { return 64 * SUB; }
@@ -191,7 +253,7 @@ struct BPiece<GGML_Q8_0> : NoLookup<BPiece<GGML_Q8_0>> {
   __device__ __forceinline__ static void load_hp(const uint8_t* row, int sb, int h, int p, const uint32_t*, Raw& r) {
     const uint8_t* b = row + (8 * sb + 4 * S2 + 2 * p + h) * QB8_0;
     const uint32_t* a = dword_floor(b);
-    r.s = byte_shift(b);  // 0 or 2
+    r.s = byte_shift(b);
     const u32x4_t w0 = M::template ld<u32x4_a4_t>(a), w1 = M::template ld<u32x4_a4_t>(a + 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -200,16 +262,27 @@ struct BPiece<GGML_Q8_0> : NoLookup<BPiece<GGML_Q8_0>> {
     }
     r.w[8] = M::template ld<uint32_t>(a + 8);
   }
-  template <int S2>
+  template <int S2, bool SZ = false>
   __device__ __forceinline__ static void decode_hp(const Head&, const Raw& r, const uint32_t*, int, uint32_t out[16]) {
-    const float d = half_bits_to_float(r.s ? (r.w[0] >> 16) : (r.w[0] & 0xFFFF));
+    const float d = half_bits_to_float((uint16_t)(r.s ? r.w[0] >> 16 : r.w[0] & 0xFFFFu));
+    if constexpr (SZ) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t q = r.s ? r.w[i + 1] : alignbyte(r.w[i + 1], r.w[i], 2);
+        out[2 * i] = f2bf2(d * (float)(int8_t)(q & 0xFF), d * (float)(int8_t)((q >> 8) & 0xFF));
+        out[2 * i + 1] = f2bf2(d * (float)(int8_t)((q >> 16) & 0xFF), d * (float)(int8_t)(q >> 24));
+      }
+      return;
+    }
+    // d q = d (q + 128) - 128 d, exact before its one rounding (to bf16). The block's codes
+    // start 2 bytes past its d: bytes 0 and 2 of word i are bytes 2 and 4 (s = 0) or 4 and 6
+    // (s = 2) of the dword pair i, i + 1
+    const float dn = d * kCodeScale, c = -128.0f * d;
+    const uint32_t even = r.s ? 0x0C060C04u : 0x0C040C02u, odd = even + 0x00010001u;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const uint32_t q = r.s ? r.w[i + 1] : alignbyte(r.w[i + 1], r.w[i], 2);
-      const float y0 = d * (float)(int8_t)(q & 0xFF), y1 = d * (float)(int8_t)((q >> 8) & 0xFF);
-      const float y2 = d * (float)(int8_t)((q >> 16) & 0xFF), y3 = d * (float)(int8_t)(q >> 24);
-      out[2 * i] = f2bf2(y0, y1);
-      out[2 * i + 1] = f2bf2(y2, y3);
+      const uint32_t lo = r.w[i] ^ 0x80808080u, hi = r.w[i + 1] ^ 0x80808080u;
+      codes4(dn, c, __builtin_amdgcn_perm(hi, lo, even), __builtin_amdgcn_perm(hi, lo, odd), out + 2 * i);
     }
   }
   __device__ static int off0(int h) { return 32 * h; }
@@ -218,16 +291,14 @@ struct BPiece<GGML_Q8_0> : NoLookup<BPiece<GGML_Q8_0>> {
 
 template <>
 struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
-  static constexpr int NLOAD = 4;  // VMEM instructions per load<SUB>, at least
+  static constexpr int NLOAD = 2;  // VMEM instructions per load<SUB>, at least
   // VMEM instructions of load_next over two consecutive steps: the odd step of a pair loads
   // only its ql bytes (the pair's qh bytes are the same)
-  static constexpr int NLOAD2 = 6;
-  // VALU instructions the GEMM schedule places after each MFMA: 4 for a decode of 4.1 a MFMA
-  // (headline down GEMM 255 -> 250 us at the sustained clock; 5 and 6 slower, 3 no better)
+  static constexpr int NLOAD2 = 3;
+  // VALU instructions the GEMM schedule places after each MFMA
   static constexpr int VPM = 4;
-  // the 20 bytes from the dword below scales[0]: scales[16] and d, s = byte shift
-  struct Head { uint32_t w[5]; uint32_t s; };
-  struct Raw { uint32_t ql[5], qh[5]; };
+  struct Head { uint32_t sc[4]; uint32_t d; };  // scales[16] and d
+  struct Raw { uint32_t ql[4], qh[4]; };
   template <int SUB>
   __device__ static int ksub() { return 128 * (SUB >> 1) + 32 * (SUB & 1); }
   template <int S2>
@@ -236,29 +307,14 @@ struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
   template <class M = GMem>
   __device__ static void load_head(const uint8_t* row, int sb, int, Head& hd) {
     const uint8_t* sc = row + sb * QB6_K + 192;
-    hd.s = byte_shift(sc);
-    const uint32_t* a = dword_floor(sc);
-    const u32x4_t w = M::template ld<u32x4_a4_t>(a);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) hd.w[i] = w[i];
-    hd.w[4] = M::template ld<uint32_t>(a + 4);
+    M::template words<4>(sc, hd.sc);
+    hd.d = M::template ld<uint16_t>(sc + 16);
   }
   template <int S2, class M = GMem>
   __device__ __forceinline__ static void load_hp(const uint8_t* row, int sb, int h, int p, const uint32_t*, Raw& r) {
     const uint8_t* b = row + sb * QB6_K;
-    constexpr int hh = S2;
-    const int c = p;
-    const uint32_t* ql = dword_floor(b + 64 * hh + 32 * c + 16 * h);
-    const uint32_t* qh = dword_floor(b + 128 + 32 * hh + 16 * h);
-    // 16 bytes each from the dword below them: one dwordx4 and the dword after it
-    const u32x4_t l4 = M::template ld<u32x4_a4_t>(ql), h4 = M::template ld<u32x4_a4_t>(qh);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      r.ql[i] = l4[i];
-      r.qh[i] = h4[i];
-    }
-    r.ql[4] = M::template ld<uint32_t>(ql + 4);
-    r.qh[4] = M::template ld<uint32_t>(qh + 4);
+    M::template words<4>(b + 64 * S2 + 32 * p + 16 * h, r.ql);
+    M::template words<4>(b + 128 + 32 * S2 + 16 * h, r.qh);
   }
   // steps 2 hh and 2 hh + 1 read the same 16 qh bytes (bits 2c.. of run c, c = SUB & 1): the
   // odd step takes them from the even one's raw bytes and loads only its ql bytes
@@ -268,47 +324,49 @@ struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
     if constexpr ((SUB & 1) == 0) {
       load_hp<SUB / 2>(row, sb, h, 0, grid, r);
     } else {
-      const uint32_t* ql = dword_floor(row + sb * QB6_K + 64 * (SUB / 2) + 32 + 16 * h);
-      const u32x4_t l4 = GMem::ld<u32x4_a4_t>(ql);
+      GMem::words<4>(row + sb * QB6_K + 64 * (SUB / 2) + 32 + 16 * h, r.ql);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) r.ql[i] = l4[i];
-      r.ql[4] = GMem::ld<uint32_t>(ql + 4);
-#pragma unroll
-      for (int i = 0; i < 5; ++i) r.qh[i] = prev.qh[i];
+      for (int i = 0; i < 4; ++i) r.qh[i] = prev.qh[i];
     }
   }
-  template <int S2>
+  template <int S2, bool SZ = false>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t*, int p,
                                                    uint32_t out[16]) {
     constexpr int hh = S2;
     const int c = p;
-    const uint32_t s = hd.s;  // the same shift as the block start (192 = 0 mod 4)
     // scales[8hh + 2c + h] (run c) and scales[8hh + 2c + h + 4] (run c+2): bytes 2c + h of
-    // the realigned scale words 2hh and 2hh + 1
+    // scale words 2hh and 2hh + 1
     const uint32_t h8 = 8 * ((threadIdx.x >> 5) & 1);
-    const uint32_t sa = alignbyte(hd.w[2 * hh + 1], hd.w[2 * hh], s);
-    const uint32_t sbw = alignbyte(hd.w[2 * hh + 2], hd.w[2 * hh + 1], s);
-    const float d = half_bits_to_float(alignbyte(hd.w[4], hd.w[4], s) & 0xFFFF);
-    // y = (d sc) (q - 32) as the product of (d sc / 4), exact, and the signed byte 4 (q - 32),
-    // converted with one v_cvt_f32_i32 (sdwa, sign-extended byte): one rounding of the exact
-    // product, and the signed zeros of a plain multiply (q = 32 under a negative scale
-    // gives -0, as (d sc) * 0 does). The 6-bit code q - 32 is q with its bit 5 flipped, read
-    // as 6-bit two's complement: flipping bits 1, 3, 5, 7 of every qh byte flips bit 5 of
-    // both runs' codes; the code then sits in bits 2..7 of its byte.
-    const float d1a = 0.25f * (d * (float)(int8_t)((sa >> (16 * c + h8)) & 0xFF));
-    const float d1b = 0.25f * (d * (float)(int8_t)((sbw >> (16 * c + h8)) & 0xFF));
+    const uint32_t sa = hd.sc[2 * hh], sbw = hd.sc[2 * hh + 1];
+    const float d = half_bits_to_float((uint16_t)hd.d);
+    const float fa = d * (float)(int8_t)((sa >> (16 * c + h8)) & 0xFF);
+    const float fb = d * (float)(int8_t)((sbw >> (16 * c + h8)) & 0xFF);
     const int hsh = 2 * c;
+    // run c: low nibbles and qh bits hsh, hsh+1; run c+2: high nibbles and bits hsh+4, hsh+5
+    if constexpr (SZ) {
+      // the product of (d sc / 4), exact, and the signed byte 4 (q - 32): q with bit 5 flipped
+      // (bits 1, 3, 5, 7 of every qh byte) is a 6-bit two's complement number, in bits 2..7
+      const float qa = 0.25f * fa, qb = 0.25f * fb;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t hx = r.qh[i] ^ 0xAAAAAAAAu;
+        const uint32_t va = bfi(0xC0C0C0C0u, hx << (6 - hsh), (r.ql[i] & 0x0F0F0F0Fu) << 2);
+        const uint32_t vb = bfi(0xC0C0C0C0u, hx << (2 - hsh), (r.ql[i] >> 2) & 0x3C3C3C3Cu);
+        out[2 * i] = f2bf2(qa * (float)(int8_t)(va & 0xFF), qa * (float)(int8_t)((va >> 8) & 0xFF));
+        out[2 * i + 1] = f2bf2(qa * (float)(int8_t)((va >> 16) & 0xFF), qa * (float)(int8_t)(va >> 24));
+        out[8 + 2 * i] = f2bf2(qb * (float)(int8_t)(vb & 0xFF), qb * (float)(int8_t)((vb >> 8) & 0xFF));
+        out[8 + 2 * i + 1] = f2bf2(qb * (float)(int8_t)((vb >> 16) & 0xFF), qb * (float)(int8_t)(vb >> 24));
+      }
+      return;
+    }
+    // (d sc) (q - 32) = (d sc) q - 32 (d sc): one rounding of the exact value (32 (d sc) is exact)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t lw = alignbyte(r.ql[i + 1], r.ql[i], s);
-      const uint32_t hw = alignbyte(r.qh[i + 1], r.qh[i], s) ^ 0xAAAAAAAAu;
-      // run c: low nibbles and qh bits hsh, hsh+1; run c+2: high nibbles and bits hsh+4, hsh+5
-      const uint32_t va = bfi(0xC0C0C0C0u, hw << (6 - hsh), (lw & 0x0F0F0F0Fu) << 2);
-      const uint32_t vb = bfi(0xC0C0C0C0u, hw << (2 - hsh), (lw >> 2) & 0x3C3C3C3Cu);
-      out[2 * i] = f2bf2(d1a * (float)(int8_t)(va & 0xFF), d1a * (float)(int8_t)((va >> 8) & 0xFF));
-      out[2 * i + 1] = f2bf2(d1a * (float)(int8_t)((va >> 16) & 0xFF), d1a * (float)(int8_t)(va >> 24));
-      out[8 + 2 * i] = f2bf2(d1b * (float)(int8_t)(vb & 0xFF), d1b * (float)(int8_t)((vb >> 8) & 0xFF));
-      out[8 + 2 * i + 1] = f2bf2(d1b * (float)(int8_t)((vb >> 16) & 0xFF), d1b * (float)(int8_t)(vb >> 24));
+      const uint32_t lw = r.ql[i], hw = r.qh[i];
+      // bits 6 and 7 of the bytes are others' and masked off with the split into half-words
+      const uint32_t va = bfi(0x0F0F0F0Fu, lw, hw << (4 - hsh)), vb = bfi(0x0F0F0F0Fu, lw >> 4, hw >> hsh);
+      codes4(fa * kCodeScale, -32.0f * fa, and_opaque(va, 0x003F003Fu), and_opaque(va >> 8, 0x003F003Fu), out + 2 * i);
+      codes4(fb * kCodeScale, -32.0f * fb, and_opaque(vb, 0x003F003Fu), and_opaque(vb >> 8, 0x003F003Fu), out + 8 + 2 * i);
     }
   }
   __device__ static int off0(int h) { return 16 * h; }
@@ -318,15 +376,13 @@ struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
 template <>
 struct BPiece<GGML_IQ3_S> {
   // `grid` is the codebook as byte selectors, staged in LDS by stage_iq3s_sel (formats.h).
-  // VMEM instructions per load<SUB>: qs (dwordx2 + dword, merged into one dwordx3), the
-  // signs (dwordx2) and the qh dword
-  static constexpr int NLOAD = 3;
-  static constexpr int NLOAD2 = 6;  // VMEM instructions of load_next over two consecutive steps
+  static constexpr int NLOAD = 2;  // VMEM instructions per load<SUB>: qs and the signs
+  static constexpr int NLOAD2 = 4;  // VMEM instructions of load_next over two consecutive steps
   static constexpr int VPM = 4;    // VALU instructions the GEMM schedule places after each MFMA
-  // d and the 4 scale bytes of the block (dwords below them, realigned at decode)
-  struct Head { uint32_t dw, sc0, sc1; uint32_t s; };
-  // qs[8] of group ib (3 dwords from below), qh byte's dword, signs[4] (2 dwords from below)
-  struct Raw { uint32_t qs[3], sg[2], qh; };
+  // d, the 4 scale bytes and the 8 qh bytes of the block
+  struct Head { uint32_t d, sc, qh[2]; };
+  // qs[8] and signs[4] of group ib
+  struct Raw { uint32_t qs[2], sg; };
   template <int SUB>
   __device__ static int ksub() { return 64 * SUB; }
   template <int S2>
@@ -335,37 +391,25 @@ struct BPiece<GGML_IQ3_S> {
   template <class M = GMem>
   __device__ static void load_head(const uint8_t* row, int sb, int, Head& hd) {
     const uint8_t* b = row + sb * QBIQ3_S;
-    hd.s = byte_shift(b);
-    hd.dw = M::template ld<uint32_t>(dword_floor(b));
-    hd.sc0 = M::template ld<uint32_t>(dword_floor(b + 106));
-    hd.sc1 = M::template ld<uint32_t>(dword_floor(b + 108));
+    hd.d = M::template ld<uint16_t>(b);
+    M::template words<2>(b + 66, hd.qh);
+    M::template words<1>(b + 106, &hd.sc);
   }
   template <int S2, class M = GMem>
   __device__ __forceinline__ static void load_hp(const uint8_t* row, int sb, int h, int p, const uint32_t*, Raw& r) {
     const uint8_t* b = row + sb * QBIQ3_S;
     const int ib = 4 * S2 + 2 * p + h;
-    const uint32_t* q = dword_floor(b + 2 + 8 * ib);
-    const u32x2_t q2 = M::template ld<u32x2_a4_t>(q);
-    r.qs[0] = q2[0];
-    r.qs[1] = q2[1];
-    r.qs[2] = M::template ld<uint32_t>(q + 2);
-    const u32x2_t s2 = M::template ld<u32x2_a4_t>(dword_floor(b + 74 + 4 * ib));
-    r.sg[0] = s2[0];
-    r.sg[1] = s2[1];
-    r.qh = M::template ld<uint32_t>(dword_floor(b + 66 + ib));
+    M::template words<2>(b + 2 + 8 * ib, r.qs);
+    M::template words<1>(b + 74 + 4 * ib, &r.sg);
   }
   // the 8 codebook entries of the piece's 4-value groups
   struct Look { uint32_t g[8]; };
   template <int S2>
   __device__ __forceinline__ static void lookup_hp(const Head& hd, const Raw& r, const uint32_t* grid, int p,
                                                    Look& lk) {
-    const uint32_t s = hd.s;
     const uint32_t h = (threadIdx.x >> 5) & 1;
-    const int ib = 4 * S2 + 2 * p + (int)h;
-    // block byte offsets: qs at 2 + 8 ib (= s + 2 mod 4), qh at 66 + ib
-    const uint32_t s2 = (s + 2) & 3;
-    const uint32_t qs0 = alignbyte(r.qs[1], r.qs[0], s2), qs1 = alignbyte(r.qs[2], r.qs[1], s2);
-    const uint32_t qh = __builtin_amdgcn_ubfe(r.qh, 8 * ((s + 2 + ib) & 3), 8);
+    const uint32_t qs0 = r.qs[0], qs1 = r.qs[1];
+    const uint32_t qh = __builtin_amdgcn_ubfe(hd.qh[S2], 8 * (2 * (uint32_t)p + h), 8);  // qh byte 4 S2 + 2p + h
     const uint32_t qh2 = qh | (qh << 16);
     // the 9-bit indices of groups 2j and 2j + 1 as the two 16-bit halves of one word: their
     // qs bytes moved to bits 0 and 16 by one v_perm, qh bits 2j and 2j + 1 to bits 8 and 24
@@ -385,16 +429,11 @@ struct BPiece<GGML_IQ3_S> {
   template <int S2>
   __device__ __forceinline__ static void convert_hp(const Head& hd, const Raw& r, const uint32_t*, int p,
                                                     const Look& lk, uint32_t out[16]) {
-    const uint32_t s = hd.s;
     const uint32_t h = (threadIdx.x >> 5) & 1;
-    const int ib = 4 * S2 + 2 * p + (int)h;
-    // block byte offsets: signs at 74 + 4 ib (= s + 2 mod 4), scales at 106, d at 0
-    const uint32_t s2 = (s + 2) & 3;
-    const uint32_t sg = alignbyte(r.sg[1], r.sg[0], s2);
-    const uint32_t scw = alignbyte(hd.sc1, hd.sc0, s2);  // scales[0..3]
-    const uint32_t nib = (scw >> (8 * (ib >> 1) + 4 * (ib & 1))) & 15;
-    const uint32_t dbits = (hd.dw >> (8 * s)) & 0xFFFF;
-    const float db = half_bits_to_float(dbits) * (float)(1 + 2 * (int)nib);
+    const uint32_t sg = r.sg;
+    const uint32_t nib = (hd.sc >> (8 * (2 * S2 + p) + 4 * h)) & 15;  // group 4 S2 + 2p + h
+    const uint32_t dbits = hd.d;
+    const float db = half_bits_to_float((uint16_t)dbits) * (float)(1 + 2 * (int)nib);
     // A group has only eight magnitudes m = 2e + 1: bf16(db * m) of each (the same rounding
     // of the same exact product as a value-by-value decode) goes into a table of two byte
     // planes, byte e of {tl1:tl0} the low byte of entry e, of {th1:th0} its high byte. The
@@ -426,7 +465,7 @@ struct BPiece<GGML_IQ3_S> {
       out[2 * k + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u) ^ pair_signs(2 * k + 1);
     }
   }
-  template <int S2>
+  template <int S2, bool SZ = false>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t* grid, int p,
                                                    uint32_t out[16]) {
     Look lk;

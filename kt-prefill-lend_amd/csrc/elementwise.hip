@@ -51,25 +51,29 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
     r = r0 + dr;
     sb = (int)(t - dr * (uint32_t)nsb);
   };
+  // a lane past the last unit reads the last one (its values are not stored): no branch, so that
+  // every load is on its way before the first is waited for
   int64_t r;
   int sb;
-  place(ul, r, sb);
+  place((int)(u0 + ul < total ? ul : total - 1 - u0), r, sb);
   const uint8_t* row = raw + e * raw_stride + r * rb;
-  const bool live = u0 + ul < total;
   typename BP::Head hd;
   typename BP::Raw rw[2];
   // Q8_0 rows may end inside a column (a piece is one 32-value block): the pieces past the
   // row's end are not loaded
-  auto inside = [&](int ks) { return live && 256 * (int64_t)sb + ks + BP::off0(h) < cols; };
-  if (live) BP::load_head(row, sb, h, hd);
+  auto inside = [&](int ks) {
+    return TYPE != GGML_Q8_0 || 256 * (int64_t)sb + ks + BP::off0(h) < cols;
+  };
+  BP::load_head(row, sb, h, hd);
   if (inside(BP::template ksub_hp<0>(p))) BP::template load_hp<0>(row, sb, h, p, grid, rw[0]);
   if (inside(BP::template ksub_hp<1>(p))) BP::template load_hp<1>(row, sb, h, p, grid, rw[1]);
+  __builtin_amdgcn_sched_barrier(0);  // (67 us without it)
   uint8_t* stg = stage + wave * DQ_STG;
   uint16_t* oe = out + e * out_stride;
   auto half = [&](auto s2c) {
     constexpr int S2 = decltype(s2c)::value;
     uint32_t v[16];
-    BP::template decode_hp<S2>(hd, rw[S2], grid, p, v);
+    BP::template decode_hp<S2, true>(hd, rw[S2], grid, p, v);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const int q = c < 2 ? BP::off0(h) / 8 + c : BP::off1(h) / 8 + c - 2;

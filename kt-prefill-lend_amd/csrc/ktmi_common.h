@@ -32,6 +32,10 @@ typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 // read from the dword below them)
 typedef uint32_t u32x4_a4_t __attribute__((ext_vector_type(4))) __attribute__((aligned(4)));
 typedef uint32_t u32x2_a4_t __attribute__((ext_vector_type(2))) __attribute__((aligned(4)));
+// and with 2-byte alignment: global loads take any address
+typedef uint32_t u32x4_a2_t __attribute__((ext_vector_type(4))) __attribute__((aligned(2)));
+typedef uint32_t u32x2_a2_t __attribute__((ext_vector_type(2))) __attribute__((aligned(2)));
+typedef uint32_t u32_a2_t __attribute__((aligned(2)));
 
 namespace ktmi {
 

@@ -386,10 +386,12 @@ constexpr int wait_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) 
 // are free of bank conflicts.
 __device__ __forceinline__ int lds_slot(int row, int chunk) { return chunk ^ (row & 7) ^ ((row >> 3) & 1); }
 
-// 128-route tiles of the light decodes (Q8_0, Q4_K) fit two waves per SIMD (accumulators in
-// VGPRs, 256 registers a lane), so two blocks share a CU; Q6_K and IQ3_S would spill there.
+// 128-route tiles fit two waves per SIMD (accumulators in VGPRs, 256 registers a lane), so two
+// blocks share a CU. IQ3_S spills 13 to 20 registers for it and still gains (2047 tokens of the
+// 2048 x 512 layer with 48 slots: 207 -> 192 us a layer); Q6_K stays at one (10 spilled:
+// 7168 x 2048 down, 300 tokens: 325 -> 335 us).
 template <int TYPE, int FJ>
-constexpr int gemm_waves_per_simd() { return FJ == 8 || TYPE == GGML_Q6_K || TYPE == GGML_IQ3_S ? 1 : 2; }
+constexpr int gemm_waves_per_simd() { return FJ == 8 || TYPE == GGML_Q6_K ? 1 : 2; }
 
 // GATEUP = true : activations = x rows gathered through perm (here the sorted routes' tokens),
 //                 Kdim = hidden, weight rows = [gate n0.. ; up NI+n0..], out = H [R, NI]
@@ -647,9 +649,10 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const uint16_t* __restr
       // schedule: the direct loads first, then 32 x (1 MFMA, VPM VALU), an LDS read after
       // every other MFMA and one of the raw weight gathers after every other (each
       // gathers 32 rows' cache lines: in one burst they would hold up the MFMA issue).
-      // VPM covers the type's decode (Q4_K and Q8_0 about 3.5 VALU per MFMA, Q6_K 4.1,
-      // IQ3_S 4.3 once its codebook reads are out of the region): VALU left over would run
-      // after the last MFMA with the matrix core idle.
+      // VPM covers the type's decode at 256-route tiles (Q4_K and Q8_0 about 2.8 VALU per MFMA,
+      // Q6_K 3.2, IQ3_S 3.5): VALU left over would run after the last MFMA with the matrix
+      // core idle. (128-route tiles have twice that per MFMA; placing 6 to 8 there made no
+      // difference.)
       // (gate/up: the direct loads take the first of the per-MFMA VMEM slots instead of a
       // burst at the region's start: gate/up 337.5 -> 335.5 us at the sustained clock; the
       // down GEMM unchanged either way)

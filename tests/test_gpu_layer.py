@@ -505,3 +505,31 @@ def test_fused_decode_down_units(dev, types, inter):
     exp = R.bf16_to_f32(gemv_layer_oracle(xb, tw, slot, w13, w2, w.types, w.hidden, w.inter))
     l2, _, _ = R.rel_errors(got, exp)
     assert l2 < 4e-3, l2
+
+
+@pytest.mark.parametrize("t", [R.GGML_Q8_0, R.GGML_Q4_K, R.GGML_Q6_K, R.GGML_IQ3_S])
+@pytest.mark.parametrize("T,mode", [(7, "decode"), (70, "grouped"), (300, "grouped")])
+def test_matrix_decoders_over_all_codes(dev, t, T, mode):
+    """The matrix kernels' decoders on blocks of random codes and scales with negative, zero and
+    the smallest fp16 scales among them, against the fp64 FFN on the exact values."""
+    L, _, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=512, inter=256, hot=5, experts=16, types=(t, t, t))
+    rng = np.random.default_rng(t)
+    _, tw, slot, _ = S.routing(w, T)
+    xb = S.activations(w, T)
+    size, at = {R.GGML_Q8_0: (34, (0,)), R.GGML_Q4_K: (144, (0, 2)), R.GGML_Q6_K: (210, (208,)), R.GGML_IQ3_S: (110, (0,))}[t]
+
+    def blocks(a):
+        b = rng.integers(0, 256, size=a.shape, dtype=np.uint8).reshape(-1, size)
+        for o in at:
+            d = (rng.random(b.shape[0]) * 2e-4 * rng.choice([-1.0, 1.0], b.shape[0])).astype(np.float16)
+            d[::7], d[3::11] = 0.0, np.float16(6e-8)
+            b[:, o:o + 2] = d.view(np.uint8).reshape(-1, 2)
+        return b.reshape(a.shape)
+
+    w13, w2 = (blocks(a) for a in S.slot_tensors(w))
+    got = R.bf16_to_f32(_run(dev, w, xb, tw, slot, w13, w2, L.MODE_DECODE if mode == "decode" else L.MODE_GROUPED))
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    l2, l1, cos = R.rel_errors(got, R.ffn_reference(xb, slot, tw, g, d))
+    assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
