@@ -103,9 +103,18 @@ __global__ __launch_bounds__(256) void moe_gemv_kernel(const uint8_t* __restrict
     for (int r = rbase + threadIdx.x; r < rbase + BR && r < rows; r += blockDim.x) Y[(int64_t)p * rows + r] = cvt_out<OutT>(0.0f);
     return;
   }
+  // the routes of this expert, 64 ids a load and ballot. One id after the other, each a round
+  // trip to the cache, this was most of a larger window's time: 32 tokens x top-10 of 1536 x 2048
+  // Q8_0 432 -> 92 us, 6 tokens x top-8 of 7168 x 2048 Q4_K 90 -> 62.
+  const int lane = threadIdx.x & 63;
+  auto same = [&](int b) { return __ballot(b + lane < n_routes && ids[min(b + lane, n_routes - 1)] == e); };
+  int base = p & ~63;
+  uint64_t m = 0;
   if (!per_route) {
-    for (int q = 0; q < p; ++q)
-      if (ids[q] == e) return;  // an earlier route of this expert computes this one
+    for (int b = 0; b < base; b += 64)
+      if (same(b)) return;  // an earlier route of this expert computes this one
+    m = same(base);
+    if (m & ((1ull << (p & 63)) - 1)) return;
   }
   if constexpr (TYPE == GGML_IQ3_S) {
     stage_iq3s_grid(grid);
@@ -113,17 +122,24 @@ __global__ __launch_bounds__(256) void moe_gemv_kernel(const uint8_t* __restrict
   }
   const int64_t rb = row_bytes(cols, TYPE);
   const uint8_t* wexp = w_is_table ? (const uint8_t*)((const int64_t*)W)[e] : W + (int64_t)e * w_expert_stride;
-  int q = p;
   while (true) {
-    int mem[4];
+    int mem[4] = {p, p, p, p};
     int nm = 0;
     if (per_route) {
-      if (q != p) break;
-      mem[nm++] = p;
-      q = n_routes;
+      nm = 1;
     } else {
-      for (; q < n_routes && nm < 4; ++q)
-        if (ids[q] == e) mem[nm++] = q;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {  // uniform: the next route in ascending order
+        while (m == 0 && base + 64 < n_routes) {
+          base += 64;
+          m = same(base);
+        }
+        if (m) {
+          mem[j] = base + (int)__builtin_ctzll(m);
+          m &= m - 1;
+          nm = j + 1;
+        }
+      }
     }
     if (nm == 0) break;
     switch (nm) {

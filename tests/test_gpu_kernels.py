@@ -113,6 +113,26 @@ def test_moe_a8_vec(dev, t, per_route):
     assert R.rel_errors(got, ref)[0] < 5e-3
 
 
+@pytest.mark.parametrize("t", [R.GGML_Q4_K, R.GGML_IQ3_S])
+@pytest.mark.parametrize("tokens,top_k", [(63, 1), (8, 8), (13, 5), (26, 10)])
+def test_moe_a8_vec_members_past_64_routes(dev, t, tokens, top_k):
+    """The routes of an expert are found 64 at a time: 63, 64, 65 and 260 routes, experts whose
+    first route is the last of a 64 or past it, and more than four of one expert, give the
+    per-route kernel's rows bit for bit."""
+    import torch
+
+    _, M, _, _ = _pkg()
+    rng = np.random.default_rng(tokens)
+    E, rows, cols = 7, 40, 512
+    W = to_dev(np.stack([random_blocks(t, rows, cols, rng) for _ in range(E)]), dev)
+    ids = rng.integers(-1, 5, size=tokens * top_k).astype(np.int32)
+    ids[62:63], ids[63:66], ids[-1:] = 5, 6, 5
+    x = bf16_tensor(R.bf16_bits(rng.standard_normal((tokens, cols)).astype(np.float32)), dev)
+    got, ref = (f(x, W, to_dev(ids, dev), top_k, t, rows, tokens) for f in (M.moe_a8_vec_multi, M.moe_a8_vec_routes))
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits_of(got), bf16_bits_of(ref))
+
+
 def test_moe_a8_vec_pointer_table(dev):
     """W as an int64 table of per-slot addresses gives the slot tensor's sums."""
     import torch
