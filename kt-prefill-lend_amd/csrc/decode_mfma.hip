@@ -572,13 +572,20 @@ bool decode_mfma_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
   return window_shape(L) && tokens * top_k <= DM_MAX_ROUTES && tokens <= DM_MAX_TOKENS;
 }
 
-// The chunks the grouped mode gives to these kernels: at 40 tokens they take 42 / 53 / 58 / 148 us
-// (2048 x 768 Q8_0 with 16 slots, 2048 x 512 Q4_K/Q6_K with 40, 2048 x 512 IQ3_S with 48,
-// 7168 x 2048 Q4_K with 16) against the grouped GEMMs' 61 / 67 / 78 / 192; at 77 tokens 54 / 61 /
-// 78 against 60 / 67 / 80, at 128 tokens they are slower on every one: a slot's x and h rows,
-// one 16-byte piece a lane from 16 rows at a time, are then what their loads are busy with.
+// The chunks the grouped mode gives to these kernels. Up to 64 tokens a slot's routes share one
+// pass over its weights, and at 40 tokens they take 42 / 53 / 58 / 148 us (2048 x 768 Q8_0 with
+// 16 slots, 2048 x 512 Q4_K/Q6_K with 40, 2048 x 512 IQ3_S with 48, 7168 x 2048 Q4_K with 16)
+// against the grouped GEMMs' 61 / 67 / 78 / 192, whose blocks pay for 128 routes a slot. Up to
+// 128 tokens only the popular slots need a second pass, and it depends on the routes a slot
+// (counting the cold ones): at 8 to 17 they take 54-57 against 69 us (2048 x 768 Q4_K, 40 slots),
+// 98-110 against 156 (4096 x 1024 Q8_0, 24), 228-254 against 313-324 (7168 x 2048 Q4_K/Q6_K, 24),
+// 249 against 487 (7168 x 2048 Q8_0, 20), 60 against 64 (2048 x 512 Q4_K/Q6_K, 40, 77 tokens); at
+// 20 to 27 66 against 65 and 73 against 66 (the same layer, 100 and 128 tokens), at 35 to 64
+// 227-347 against 208-212 (7168 x 2048, 16): a slot's x and h rows, one 16-byte piece a lane
+// from 16 rows at a time, are then what their loads are busy with.
 bool window_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
-  return window_shape(L) && tokens * top_k <= DM_ROUTES && tokens <= 64;
+  const int64_t R = tokens * top_k;
+  return window_shape(L) && R <= DM_ROUTES && (tokens <= 64 || (tokens <= 128 && R <= 18 * L->n_slots));
 }
 
 namespace {

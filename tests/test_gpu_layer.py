@@ -533,3 +533,26 @@ def test_matrix_decoders_over_all_codes(dev, t, T, mode):
     g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
     l2, l1, cos = R.rel_errors(got, R.ffn_reference(xb, slot, tw, g, d))
     assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
+
+
+@pytest.mark.parametrize("types", [(R.GGML_Q4_K, R.GGML_Q6_K), (R.GGML_Q8_0, R.GGML_IQ3_S)])
+@pytest.mark.parametrize("T,top_k,hot", [(65, 4, 15), (65, 4, 14), (128, 8, 57), (128, 8, 56), (129, 2, 40)])
+def test_window_limits(dev, types, T, top_k, hot):
+    """The grouped mode on both sides of the line between the decode-sized kernels and the
+    GEMMs (128 tokens, 18 routes a slot, 1024 routes), one slot on every token (several passes
+    of 64 routes); against the fp64 FFN."""
+    L, _, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=512, inter=256, hot=hot, experts=128, top_k=top_k, types=(types[0], types[0], types[1]))
+    rng = np.random.default_rng(T + hot)
+    slot = rng.integers(0, 2 * hot, size=(T, top_k)).astype(np.int32)
+    slot = np.where(slot < hot, slot, -1).astype(np.int32)
+    slot[:, 0] = 3
+    tw = rng.random((T, top_k)).astype(np.float32)
+    tw /= tw.sum(axis=1, keepdims=True)
+    xb = S.activations(w, T)
+    w13, w2 = S.slot_tensors(w)
+    got = R.bf16_to_f32(_run(dev, w, xb, tw, slot, w13, w2, L.MODE_GROUPED))
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    l2, l1, cos = R.rel_errors(got, R.ffn_reference(xb, slot, tw, g, d))
+    assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
