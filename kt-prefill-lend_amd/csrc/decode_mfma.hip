@@ -197,7 +197,7 @@ struct ColRing {
     lds = region;
     const uint32_t mis = (uint32_t)(uintptr_t)wexp & 15u;
     base = wexp - mis;
-    bytes = (uint32_t)(rows * rb) + mis;
+    bytes = ((uint32_t)(rows * rb) + mis + 15u) & ~15u;  // whole chunks: each holds a byte of the matrix
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int q = 64 * i + lane, row = q / CH;
