@@ -209,18 +209,19 @@ struct ColRing {
   }
   // column sb into buffer buf; where more is false the same loads go past the end of a buffer
   // of no bytes (zeros, no memory access), so that the count of operations in flight does not
-  // depend on the column
+  // depend on the column. The scalar offset is 0 there too: a range check of the lane's offset
+  // against the bytes less the scalar offset would wrap with any other
   __device__ __forceinline__ void issue(int sb, int buf, bool more) const {
     const int lane = threadIdx.x & 63;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, more ? bytes : 0u, 0x00020000);
+    const int soff = ALIGNED && more ? sb * QB : 0;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int q = 64 * i + lane;
       const uint32_t o = ALIGNED ? off[i] : ((off[i] + (uint32_t)(sb * QB)) & ~15u) + 16u * (uint32_t)(q % CH);
       if ((i < NI - 1 || q < NT * DM_RT * CH) && (USED == CH || q % CH < USED))
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rsrc, (__attribute__((address_space(3))) void*)(lds + buf * BUF + 1024 * i), 16, (int)o,
-            ALIGNED ? sb * QB : 0, 0, 0);
+            rsrc, (__attribute__((address_space(3))) void*)(lds + buf * BUF + 1024 * i), 16, (int)o, soff, 0, 0);
     }
   }
   // the lane's row of tile t in buffer buf, as a row that starts at column sb

@@ -19,6 +19,9 @@ sources for gfx950 and count the instructions actually emitted.
   loads (their tiles would be past the tile's K), and the waits of its first three steps are
   checked the same way, after the loop's last iteration and after the peeled first
   super-block (a two-column tile runs no loop iteration).
+* dm_gate_up, dm_down (the decode-sized kernels' weight ring): a direct load past the last
+  column goes through a buffer of no bytes, and its scalar offset is 0 there as well, so that
+  it is out of range whichever way the scalar offset enters the range check.
 """
 import os
 import re
@@ -36,6 +39,7 @@ pytestmark = pytest.mark.skipif(not shutil.which(HIPCC) and not Path(HIPCC).exis
 
 VMEM = re.compile(r"^\s*(global_load|buffer_load)")
 DMA = re.compile(r"^\s*buffer_load\w*\s.*\blds\b")
+RING = re.compile(r"^\s*buffer_load_dwordx4 v\d+, s\[(\d+):\d+\], (\S+) offen lds")  # resource, scalar offset
 
 
 def _asm(src: str, tmp_path) -> list:
@@ -174,3 +178,32 @@ def _check_last_super_block(lines, name, a, b):
             w_at = max(i for i, l in enumerate(flat) if "s_waitcnt" in l and "vmcnt" in l)
             after = sum(1 for i in range(dmas[-1] + 1, w_at) if VMEM.match(flat[i]))
             assert 0 < _vmcnt(flat[w_at]) <= after, (name, "tail step", s, _vmcnt(flat[w_at]), after)
+
+
+@pytest.fixture(scope="module")
+def window_kernels(tmp_path_factory):
+    """{name: lines} of the decode-sized kernels: 4 types x (gate/up, down) x 5 launch shapes."""
+    lines = _asm("decode_mfma.hip", tmp_path_factory.mktemp("dm"))
+    out = {}
+    for i, l in enumerate(lines):
+        m = re.match(r"^_ZN4ktmi12_GLOBAL__N_1(10dm_gate_up|7dm_down)(ILi\d+E\w*?EEE)\w*:", l)
+        if m:
+            end = next(j for j in range(i, len(lines)) if lines[j].startswith(".Lfunc_end"))
+            out[m.group(1).lstrip("0123456789") + m.group(2)] = lines[i:end]
+    assert len(out) == 40
+    return out
+
+
+def _last_def(lines, at, reg):
+    return next(l.strip() for l in reversed(lines[:at]) if re.match(rf"\s*s_\w+ {reg},", l))
+
+
+def test_window_ring_drops_the_loads_past_the_last_column(window_kernels):
+    for name, lines in window_kernels.items():
+        loads = [(i, RING.match(l)) for i, l in enumerate(lines) if DMA.match(l)]
+        assert loads and all(m for _, m in loads), name
+        for i, m in loads:
+            soff = m.group(2)
+            if soff != "0":
+                d = _last_def(lines, i, soff)
+                assert re.match(r"s_cselect_b32 s\d+, \S+, 0$", d), (name, "scalar offset of a dropped load", lines[i].strip(), d)
