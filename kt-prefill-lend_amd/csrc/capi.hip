@@ -307,11 +307,12 @@ int ktmi_moe_layer(const ktmi_layer* L, const void* x, const float* topk_w, cons
   }
   KTMI_REQUIRE(mode == KTMI_MODE_GROUPED, KTMI_EINVAL, "moe_layer: mode %d", mode);
   const int64_t pass = grouped_pass_tokens(L, top_k);
+  const bool window = tokens <= pass && window_fits(L, tokens, top_k);
   for (int64_t t0 = 0; t0 < tokens; t0 += pass) {
     const int64_t nt = tokens - t0 < pass ? tokens - t0 : pass;
     const GroupedPlan P = grouped_plan(nt, top_k, L->n_slots, K, N);
     rc = launch_grouped_layer(L, (const uint16_t*)x + t0 * K, topk_w + t0 * top_k, slot_ids + t0 * top_k, nt, top_k,
-                              (uint16_t*)y + t0 * K, (uint8_t*)workspace, P, s);
+                              (uint16_t*)y + t0 * K, (uint8_t*)workspace, P, window, s);
     if (rc) return rc;
   }
   return KTMI_OK;

@@ -61,8 +61,10 @@ struct GroupedPlan {
   int64_t off_counts, off_seg, off_tseg, off_tinfo, off_perm, off_tok, off_h, off_y, total;
 };
 GroupedPlan grouped_plan(int64_t tokens, int64_t top_k, int64_t n_slots, int64_t hidden, int64_t inter);
+// window: run the decode-sized kernels (window_fits of the whole call, so that every pass of a
+// longer one sums in the GEMMs' order, whatever its number of tokens).
 int launch_grouped_layer(const ktmi_layer* L, const uint16_t* x, const float* topk_w, const int32_t* slot_ids,
-                         int64_t tokens, int64_t top_k, uint16_t* y, uint8_t* ws, const GroupedPlan& P,
+                         int64_t tokens, int64_t top_k, uint16_t* y, uint8_t* ws, const GroupedPlan& P, bool window,
                          hipStream_t stream);
 
 }  // namespace ktmi

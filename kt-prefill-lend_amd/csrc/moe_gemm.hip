@@ -1045,7 +1045,7 @@ GroupedPlan grouped_plan(int64_t tokens, int64_t top_k, int64_t n_slots, int64_t
 }
 
 int launch_grouped_layer(const ktmi_layer* L, const uint16_t* x, const float* topk_w, const int32_t* slot_ids,
-                         int64_t tokens, int64_t top_k, uint16_t* y, uint8_t* ws, const GroupedPlan& P,
+                         int64_t tokens, int64_t top_k, uint16_t* y, uint8_t* ws, const GroupedPlan& P, bool window,
                          hipStream_t stream) {
   const int64_t R = P.routes;
   const int S = (int)L->n_slots;
@@ -1060,7 +1060,7 @@ int launch_grouped_layer(const ktmi_layer* L, const uint16_t* x, const float* to
   KTMI_REQUIRE(tokens * K * 2 <= 0xFFFF0000ll && R * N * 2 <= 0xFFFF0000ll && R * K * 2 <= 0xFFFF0000ll, KTMI_EINVAL,
                "grouped layer: a pass of %lld tokens exceeds the 32-bit buffer range", (long long)tokens);
   if (tokens == 0) return KTMI_OK;
-  if (window_fits(L, tokens, top_k))
+  if (window)
     return launch_window(L, x, topk_w, slot_ids, tokens, top_k, y, (uint16_t*)(ws + P.off_h), (uint16_t*)(ws + P.off_y),
                          stream);
   int32_t* hist = (int32_t*)(ws + P.off_counts);

@@ -334,6 +334,32 @@ def test_grouped_past_one_pass(dev):
     assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
 
 
+def test_grouped_short_last_pass(dev):
+    """A long call whose last pass is as short as a decode window (top-64, hidden 7168: 4608
+    tokens a pass, then 12): the last tokens' outputs are those of one pass over all tokens, bit
+    for bit the ones they get at the end of a 300-token call."""
+    L, H, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=7168, inter=256, hot=4, experts=128, top_k=64)
+    desc = L.ktmi_layer(hidden=w.hidden, inter=w.inter, n_slots=w.hot, type13=w.types[0], type2=w.types[2],
+                        w13=1 << 20, w2=1 << 21)
+    cut = L.lib().ktmi_moe_layer_pass_tokens(desc, w.top_k)
+    T = cut + 12
+    assert cut == 4608
+    rng = np.random.default_rng(31)
+    slot = np.full((T, w.top_k), -1, np.int32)
+    slot[:, 5:9] = rng.integers(-1, w.hot, size=(T, 4))
+    tw = rng.random((T, w.top_k)).astype(np.float32)
+    xb = S.activations(w, T)
+    w13, w2 = S.slot_tensors(w)
+    y = _run(dev, w, xb, tw, slot, w13, w2, L.MODE_GROUPED)
+    tail = _run(dev, w, xb[-300:], tw[-300:], slot[-300:], w13, w2, L.MODE_GROUPED)
+    assert np.array_equal(y[-300:], tail)
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    l2, _, cos = R.rel_errors(R.bf16_to_f32(y[cut:]), R.ffn_reference(xb[cut:], slot[cut:], tw[cut:], g, d))
+    assert l2 < TOL_REL_L2 and cos > 0.999, (l2, cos)
+
+
 def test_grouped_at_full_shape(dev):
     """The prefill workload's real layer shape (hidden 2048, inter 512, 40 slots, Q4_K/Q6_K)
     at 1024 tokens, against the fp64 FFN on a sample of tokens."""
