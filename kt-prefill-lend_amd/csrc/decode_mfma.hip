@@ -573,20 +573,30 @@ bool decode_mfma_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
   return window_shape(L) && tokens * top_k <= DM_MAX_ROUTES && tokens <= DM_MAX_TOKENS;
 }
 
-// The chunks the grouped mode gives to these kernels. Up to 64 tokens a slot's routes share one
-// pass over its weights, and at 40 tokens they take 42 / 53 / 58 / 148 us (2048 x 768 Q8_0 with
-// 16 slots, 2048 x 512 Q4_K/Q6_K with 40, 2048 x 512 IQ3_S with 48, 7168 x 2048 Q4_K with 16)
-// against the grouped GEMMs' 61 / 67 / 78 / 192, whose blocks pay for 128 routes a slot. Up to
-// 128 tokens only the popular slots need a second pass, and it depends on the routes a slot
-// (counting the cold ones): at 8 to 17 they take 54-57 against 69 us (2048 x 768 Q4_K, 40 slots),
-// 98-110 against 156 (4096 x 1024 Q8_0, 24), 228-254 against 313-324 (7168 x 2048 Q4_K/Q6_K, 24),
-// 249 against 487 (7168 x 2048 Q8_0, 20), 60 against 64 (2048 x 512 Q4_K/Q6_K, 40, 77 tokens); at
-// 20 to 27 66 against 65 and 73 against 66 (the same layer, 100 and 128 tokens), at 35 to 64
-// 227-347 against 208-212 (7168 x 2048, 16): a slot's x and h rows, one 16-byte piece a lane
-// from 16 rows at a time, are then what their loads are busy with.
+// The chunks the grouped mode gives to these kernels instead of the GEMMs, whose blocks pay for
+// 128 routes a slot however few it has. These pay for their weights once a pass of 64 routes, and
+// their x and h rows, one 16-byte piece a lane from 16 rows at a time, grow with the routes. The
+// lines lie where they were not slower on some 900 layers drawn over types, sizes, 6 to 128 slots,
+// top-1 to top-10 and popularities, all experts in slots among them (us, these kernels against the
+// GEMMs):
+//   Q8_0 and IQ3_S in both projections (the GEMMs gather these rows a lane each): up to 64 tokens
+//     30-158 / 57-215; up to 128 with at most 18 routes a slot (counting cold ones) 110-291 /
+//     143-493, on short rows up to 640 routes (past them up to 96 / 85)
+//   with Q4_K or Q6_K: up to 40 tokens 27-109 / 49-153. Past them the GEMMs gain with every chip
+//     round (one gate/up block a CU) that their blocks fill: at most 0.7 full 57 / 64 (2048 x 512,
+//     40 slots, 77 tokens) and 205 / 304 (7168 x 2048, 20, 66); fuller, only few routes a slot
+//     (2048 x 512, 52 slots, 96 tokens 82 / 67; 7168 x 2048, 14 of 24 experts, 64 tokens 232 / 175)
+//   Q6_K gate/up: the GEMMs (2048 x 1024, 64 slots, 55 tokens 205 / 155)
 bool window_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
-  const int64_t R = tokens * top_k;
-  return window_shape(L) && R <= DM_ROUTES && (tokens <= 64 || (tokens <= 128 && R <= 18 * L->n_slots));
+  const int64_t R = tokens * top_k, S = L->n_slots;
+  if (!window_shape(L) || R > DM_ROUTES || tokens > 128 || L->type13 == GGML_Q6_K) return false;
+  if (tokens > 64 && R > 18 * S) return false;
+  const bool long_rows = L->hidden >= 4096;
+  const auto gathered = [](int t) { return t == GGML_Q8_0 || t == GGML_IQ3_S; };
+  if (gathered(L->type13) && gathered(L->type2)) return tokens <= 64 || long_rows || R <= 640;
+  const int64_t blocks = S * (L->inter / 128), rounds = (blocks + 255) / 256;
+  const int64_t most = 10 * blocks <= 7 * 256 * rounds ? (long_rows ? 40 : 64) : (long_rows ? 15 : 8);
+  return tokens <= 40 || (R <= 640 && R <= most * S);
 }
 
 namespace {

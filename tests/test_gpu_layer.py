@@ -582,3 +582,33 @@ def test_window_limits(dev, types, T, top_k, hot):
     g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
     l2, l1, cos = R.rel_errors(got, R.ffn_reference(xb, slot, tw, g, d))
     assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
+
+
+def _one_popular_slot(dev, types, hidden, inter, hot, T, top_k, mode):
+    """A call whose first slot choice is slot 3 for every token (the others spread over twice the
+    slots, half of them cold), against the fp64 FFN."""
+    _, _, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=hidden, inter=inter, hot=hot, experts=2 * hot, top_k=top_k, types=(types[0], types[0], types[1]))
+    rng = np.random.default_rng(T + hot)
+    slot = rng.integers(0, 2 * hot, size=(T, top_k)).astype(np.int32)
+    slot = np.where(slot < hot, slot, -1).astype(np.int32)
+    slot[:, 0] = 3
+    tw = rng.random((T, top_k)).astype(np.float32)
+    tw /= tw.sum(axis=1, keepdims=True)
+    xb = S.activations(w, T)
+    w13, w2 = S.slot_tensors(w)
+    got = R.bf16_to_f32(_run(dev, w, xb, tw, slot, w13, w2, mode))
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    l2, l1, cos = R.rel_errors(got, R.ffn_reference(xb, slot, tw, g, d))
+    assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
+
+
+@pytest.mark.parametrize("types", [(R.GGML_Q4_K, R.GGML_Q6_K), (R.GGML_Q6_K, R.GGML_Q4_K), (R.GGML_IQ3_S, R.GGML_Q8_0)])
+@pytest.mark.parametrize("T,top_k,hot", [(40, 16, 30), (41, 16, 30), (64, 10, 89), (64, 10, 70), (64, 8, 120), (80, 8, 89)])
+def test_window_lines(dev, types, T, top_k, hot):
+    """The grouped mode on both sides of the lines between the decode-sized kernels and the GEMMs
+    that depend on the weight types: 40 tokens, 640 routes, a chip round of gate/up blocks 0.7
+    full (89 slots of 256 rows) and the routes a slot past it."""
+    L, _, _ = _pkg()
+    _one_popular_slot(dev, types, 512, 256, hot, T, top_k, L.MODE_GROUPED)
