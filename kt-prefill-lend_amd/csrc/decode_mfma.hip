@@ -516,8 +516,16 @@ __global__ __launch_bounds__(256) void dm_combine(const uint16_t* __restrict__ y
   *(uint4*)(y + (int64_t)t * K + c) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// G (groups of 16 routes that share a pass over the weights) by the tokens, the routes a slot has unless
-// a token lists it twice; NR (ids a lane of the membership) by the routes
+// The routes a pass over a slot's weights has room for: those that the popular slots may have, at
+// most the tokens (unless a token lists a slot twice) and hardly more than eight times the mean.
+// G, the groups of 16 routes of a pass, goes by it (more groups are more registers: by the tokens
+// alone, 40 tokens x top-2 on 80 slots of the 2048 x 1024 Q6_K layer took 113 us, so 74), NR, the
+// ids a lane of the membership, by the routes
+int64_t pass_routes(int64_t tokens, int64_t R, int64_t S) {
+  const int64_t m = (8 * R + S - 1) / S;
+  return m < tokens ? m : tokens;
+}
+
 template <int TYPE>
 int launch_dm_gate_up(const ktmi_layer* L, const uint16_t* x, const int32_t* slot_ids, int64_t tokens, int64_t top_k,
                       uint16_t* hbuf, hipStream_t stream) {
@@ -529,10 +537,11 @@ int launch_dm_gate_up(const ktmi_layer* L, const uint16_t* x, const int32_t* slo
 #define KTMI_GU(G, NR)                                                                                        \
   dm_gate_up<TYPE, G, NR, 2><<<nb, DM_THREADS, 0, stream>>>(x, (int)K, (int)N, slot_ids, (int)R, (int)S, (int)top_k, \
                                                             (const uint8_t*)L->w13, L->w_is_table, st13, hbuf)
+  const int64_t m = pass_routes(tokens, R, S);
   if (R <= 256) {
-    if (tokens <= 16) KTMI_GU(1, 4); else if (tokens <= 32) KTMI_GU(2, 4); else KTMI_GU(4, 4);
+    if (m <= 16) KTMI_GU(1, 4); else if (m <= 32) KTMI_GU(2, 4); else KTMI_GU(4, 4);
   } else {
-    if (tokens <= 32) KTMI_GU(2, 16); else KTMI_GU(4, 16);
+    if (m <= 32) KTMI_GU(2, 16); else KTMI_GU(4, 16);
   }
 #undef KTMI_GU
   KTMI_HIP_TRY(hipGetLastError());
@@ -549,10 +558,11 @@ int launch_dm_down(const ktmi_layer* L, const uint16_t* hbuf, const int32_t* slo
 #define KTMI_DN(NT, G, NR)                                                                                     \
   dm_down<TYPE, NT, G, NR, 2><<<(unsigned)(S < R ? S : R) * (unsigned)(K / (64 * NT)), DM_THREADS, 0, stream>>>( \
       hbuf, (int)K, (int)N, slot_ids, (int)R, (int)S, (const uint8_t*)L->w2, L->w_is_table, st2, yv)
+  const int64_t m = pass_routes(tokens, R, S);
   if (R <= 256) {
-    if (tokens <= 16) KTMI_DN(1, 1, 4); else if (tokens <= 32) KTMI_DN(1, 2, 4); else KTMI_DN(1, 4, 4);
+    if (m <= 16) KTMI_DN(1, 1, 4); else if (m <= 32) KTMI_DN(1, 2, 4); else KTMI_DN(1, 4, 4);
   } else {
-    if (tokens <= 32) KTMI_DN(2, 2, 16); else KTMI_DN(2, 4, 16);
+    if (m <= 32) KTMI_DN(2, 2, 16); else KTMI_DN(2, 4, 16);
   }
 #undef KTMI_DN
   KTMI_HIP_TRY(hipGetLastError());

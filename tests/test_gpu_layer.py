@@ -612,3 +612,12 @@ def test_window_lines(dev, types, T, top_k, hot):
     full (89 slots of 256 rows) and the routes a slot past it."""
     L, _, _ = _pkg()
     _one_popular_slot(dev, types, 512, 256, hot, T, top_k, L.MODE_GROUPED)
+
+
+@pytest.mark.parametrize("types", [(R.GGML_Q4_K, R.GGML_Q6_K), (R.GGML_Q8_0, R.GGML_IQ3_S)])
+@pytest.mark.parametrize("T,top_k,hot,mode", [(48, 2, 70, "decode"), (60, 8, 400, "grouped")])
+def test_window_passes_follow_the_mean(dev, types, T, top_k, hot, mode):
+    """Many slots with few routes on average take passes of 16 or 32 routes although a slot on
+    every token needs several of them."""
+    L, _, _ = _pkg()
+    _one_popular_slot(dev, types, 256, 256, hot, T, top_k, L.MODE_DECODE if mode == "decode" else L.MODE_GROUPED)
