@@ -182,12 +182,17 @@ static int scratch_of_current_device(void** out) {
   return KTMI_OK;
 }
 
-// Below 64 routes the GEMV mode's two launches match or beat the decode mode's three
-// (graph-replayed steps of the 2048 x 512 Q4_K layer with 32 hot slots: 13.0 against 15.0 us at
-// 8 routes, 19.5 against 19.2 at 32); from 64 routes the decode mode's MFMAs win (23.0 against
-// 25.8 at 64, 24.2 against 30.9 at 128).
+// Below 64 routes the GEMV mode's two launches keep the reference kernels' int8 numerics at about
+// the decode mode's speed or better (graph-replayed 2048 x 512 layers with 32 hot slots, us a layer
+// GEMV / decode: Q4_K 12.7 / 13.9 at 8 routes, 19.9 / 19.1 at 32, 24.6 / 21.3 at 48; Q8_0 15.1 /
+// 17.2, 22.7 / 24.1, 28.1 / 27.6); from 64 routes the decode mode's MFMAs win (Q4_K 27.7 / 22.4 at
+// 64, 38.4 / 25.8 at 128; Q8_0 29.8 / 29.0, 39.2 / 34.7).
 // Where the rows are too long for those two launches, the decode mode starts at one route: its
-// alternative is the stage-by-stage GEMV (7168 x 2048 Q4_K/Q6_K, 40 routes: 189-244 against 87 us).
+// alternative is the stage-by-stage GEMV (7168 x 2048 Q4_K/Q6_K, 7 tokens: 164 against 60 us).
+// Above one or two routes a slot the decode mode is also the faster one on long rows of Q8_0 (2048 x
+// 512, 32 slots: the line above); with hardly one, both are bound by the weights' bytes, which the
+// GEMV's loads bring at 6.9 TB/s and the decode mode's ring at 5.3 (128 slots all hot, 16 tokens: 62
+// against 75 us). The decode mode stays there for its smaller error (0.005 against 0.0125).
 constexpr int64_t kDecodeMinRoutes = 64;
 
 int ktmi_moe_layer_mode(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
