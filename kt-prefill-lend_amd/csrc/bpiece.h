@@ -24,9 +24,8 @@
 //   Q8_0, IQ3_S: positions [32h, 32h+32) (one Q8_0 block, one IQ3_S 32-group)
 // `off0`/`off1` give the step positions of out[0..7] and out[8..15] (16 values each).
 //
-// A zero value's sign is a plain product's only with decode_hp<S2, SZ = true> (the dequant
-// entry point, whose bytes are its result: d * -0 and the like); elsewhere it may differ, which
-// no sum of products sees.
+// Zero codes and infinite or negative scales give what a plain product gives (d * -0, +-inf), in
+// every kernel: the dequant entry point, whose bytes are its result, runs the same bodies.
 //
 // Every SUB-dependent member also exists with the step parity as a run-time value: the
 // `_hp<S2>(..., p)` forms take SUB = 2 S2 + p with S2 a compile-time constant and p a
@@ -78,13 +77,29 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t b) {
 // code * 2^-24, so with d scaled by 2^24 (exact) this is the fp32 FMA of the code itself, and
 // no conversion instruction is needed. With a v_cvt a value the grouped K loop held 890 / 842 /
 // 1088 VALU a super-block column (Q4_K / Q8_0 / Q6_K, the last two with run-time realignment),
-// so 710 / 690 / 812; a 128-route block of one wave a SIMD spends half of its time issuing them
-// (2048 x 512 Q4_K/Q6_K layer, 77 tokens: 67 -> 63.5 us; 7168 x 2048, 300 tokens: 340 -> 322).
+// so 710 / 810 / 924; a 128-route block of one wave a SIMD spends half of its time issuing them
+// (2048 x 512 Q4_K/Q6_K layer, 77 tokens, in the GEMMs: 67 -> 64 us; 7168 x 2048, 300 tokens: 340 -> 322).
 constexpr float kCodeScale = 16777216.0f;  // 2^24
 template <int HI>
 __device__ __forceinline__ float fma_code(float d, uint32_t w, float c) {
   const _Float16 q = __builtin_bit_cast(_Float16, (uint16_t)(HI ? w >> 16 : w & 0xFFFFu));
   return __builtin_fmaf(d, (float)q, c);
+}
+// unsigned codes less MID in both half-words of w, as signed fp16 denormals: one v_pk_add_f16,
+// exact. Taking MID d from the FMA instead would spare it (7168 x 2048 Q8_0, 5 tokens 147 against
+// 150 us, most layers within 1 %), but give inf - inf where d is infinite and +0 for every zero
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+template <int MID>
+__device__ __forceinline__ uint32_t code_sub(uint32_t w) {
+  constexpr uint32_t m = 0x8000u | MID;
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2_t, w) + __builtin_bit_cast(f16x2_t, m | m << 16));
+}
+// -0, opaque to the compiler: an FMA with it is the plain product, signed zeros and infinities
+// included, and stays one v_fma_mix (a multiply would need a conversion)
+__device__ __forceinline__ float minus_zero() {
+  float z = -0.0f;
+  asm("" : "+s"(z));
+  return z;
 }
 // the bf16 pairs of four codes: bytes 0 and 2 of a word as the halves of e, bytes 1 and 3 of o
 __device__ __forceinline__ void codes4(float d, float c, uint32_t e, uint32_t o, uint32_t* out) {
@@ -201,7 +216,7 @@ struct BPiece<GGML_Q4_K> : NoLookup<BPiece<GGML_Q4_K>> {
   __device__ __forceinline__ static void load_hp(const uint8_t* row, int sb, int h, int p, const uint32_t*, Raw& r) {
     r.q = M::template ld<u32x4_t>(row + sb * QB4_K + 16 + 64 * S2 + 32 * p + 16 * h);
   }
-  template <int S2, bool SZ = false>
+  template <int S2>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t*, int p,
                                                    uint32_t out[16]) {
     const float d = half_bits_to_float(hd.hdr[0] & 0xFFFF);
@@ -262,27 +277,17 @@ struct BPiece<GGML_Q8_0> : NoLookup<BPiece<GGML_Q8_0>> {
     }
     r.w[8] = M::template ld<uint32_t>(a + 8);
   }
-  template <int S2, bool SZ = false>
+  template <int S2>
   __device__ __forceinline__ static void decode_hp(const Head&, const Raw& r, const uint32_t*, int, uint32_t out[16]) {
     const float d = half_bits_to_float((uint16_t)(r.s ? r.w[0] >> 16 : r.w[0] & 0xFFFFu));
-    if constexpr (SZ) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t q = r.s ? r.w[i + 1] : alignbyte(r.w[i + 1], r.w[i], 2);
-        out[2 * i] = f2bf2(d * (float)(int8_t)(q & 0xFF), d * (float)(int8_t)((q >> 8) & 0xFF));
-        out[2 * i + 1] = f2bf2(d * (float)(int8_t)((q >> 16) & 0xFF), d * (float)(int8_t)(q >> 24));
-      }
-      return;
-    }
-    // d q = d (q + 128) - 128 d, exact before its one rounding (to bf16). The block's codes
-    // start 2 bytes past its d: bytes 0 and 2 of word i are bytes 2 and 4 (s = 0) or 4 and 6
-    // (s = 2) of the dword pair i, i + 1
-    const float dn = d * kCodeScale, c = -128.0f * d;
+    // the block's codes start 2 bytes past its d: bytes 0 and 2 of word i are bytes 2 and 4
+    // (s = 0) or 4 and 6 (s = 2) of the dword pair i, i + 1
+    const float dn = d * kCodeScale;
     const uint32_t even = r.s ? 0x0C060C04u : 0x0C040C02u, odd = even + 0x00010001u;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t lo = r.w[i] ^ 0x80808080u, hi = r.w[i + 1] ^ 0x80808080u;
-      codes4(dn, c, __builtin_amdgcn_perm(hi, lo, even), __builtin_amdgcn_perm(hi, lo, odd), out + 2 * i);
+      codes4(dn, minus_zero(), code_sub<128>(__builtin_amdgcn_perm(hi, lo, even)), code_sub<128>(__builtin_amdgcn_perm(hi, lo, odd)), out + 2 * i);
     }
   }
   __device__ static int off0(int h) { return 32 * h; }
@@ -329,7 +334,7 @@ struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
       for (int i = 0; i < 4; ++i) r.qh[i] = prev.qh[i];
     }
   }
-  template <int S2, bool SZ = false>
+  template <int S2>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t*, int p,
                                                    uint32_t out[16]) {
     constexpr int hh = S2;
@@ -343,30 +348,13 @@ struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
     const float fb = d * (float)(int8_t)((sbw >> (16 * c + h8)) & 0xFF);
     const int hsh = 2 * c;
     // run c: low nibbles and qh bits hsh, hsh+1; run c+2: high nibbles and bits hsh+4, hsh+5
-    if constexpr (SZ) {
-      // the product of (d sc / 4), exact, and the signed byte 4 (q - 32): q with bit 5 flipped
-      // (bits 1, 3, 5, 7 of every qh byte) is a 6-bit two's complement number, in bits 2..7
-      const float qa = 0.25f * fa, qb = 0.25f * fb;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t hx = r.qh[i] ^ 0xAAAAAAAAu;
-        const uint32_t va = bfi(0xC0C0C0C0u, hx << (6 - hsh), (r.ql[i] & 0x0F0F0F0Fu) << 2);
-        const uint32_t vb = bfi(0xC0C0C0C0u, hx << (2 - hsh), (r.ql[i] >> 2) & 0x3C3C3C3Cu);
-        out[2 * i] = f2bf2(qa * (float)(int8_t)(va & 0xFF), qa * (float)(int8_t)((va >> 8) & 0xFF));
-        out[2 * i + 1] = f2bf2(qa * (float)(int8_t)((va >> 16) & 0xFF), qa * (float)(int8_t)(va >> 24));
-        out[8 + 2 * i] = f2bf2(qb * (float)(int8_t)(vb & 0xFF), qb * (float)(int8_t)((vb >> 8) & 0xFF));
-        out[8 + 2 * i + 1] = f2bf2(qb * (float)(int8_t)((vb >> 16) & 0xFF), qb * (float)(int8_t)(vb >> 24));
-      }
-      return;
-    }
-    // (d sc) (q - 32) = (d sc) q - 32 (d sc): one rounding of the exact value (32 (d sc) is exact)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t lw = r.ql[i], hw = r.qh[i];
       // bits 6 and 7 of the bytes are others' and masked off with the split into half-words
       const uint32_t va = bfi(0x0F0F0F0Fu, lw, hw << (4 - hsh)), vb = bfi(0x0F0F0F0Fu, lw >> 4, hw >> hsh);
-      codes4(fa * kCodeScale, -32.0f * fa, and_opaque(va, 0x003F003Fu), and_opaque(va >> 8, 0x003F003Fu), out + 2 * i);
-      codes4(fb * kCodeScale, -32.0f * fb, and_opaque(vb, 0x003F003Fu), and_opaque(vb >> 8, 0x003F003Fu), out + 8 + 2 * i);
+      codes4(fa * kCodeScale, minus_zero(), code_sub<32>(and_opaque(va, 0x003F003Fu)), code_sub<32>(and_opaque(va >> 8, 0x003F003Fu)), out + 2 * i);
+      codes4(fb * kCodeScale, minus_zero(), code_sub<32>(and_opaque(vb, 0x003F003Fu)), code_sub<32>(and_opaque(vb >> 8, 0x003F003Fu)), out + 8 + 2 * i);
     }
   }
   __device__ static int off0(int h) { return 16 * h; }
@@ -465,7 +453,7 @@ struct BPiece<GGML_IQ3_S> {
       out[2 * k + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u) ^ pair_signs(2 * k + 1);
     }
   }
-  template <int S2, bool SZ = false>
+  template <int S2>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t* grid, int p,
                                                    uint32_t out[16]) {
     Look lk;

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
   auto half = [&](auto s2c) {
     constexpr int S2 = decltype(s2c)::value;
     uint32_t v[16];
-    BP::template decode_hp<S2, true>(hd, rw[S2], grid, p, v);
+    BP::template decode_hp<S2>(hd, rw[S2], grid, p, v);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const int q = c < 2 ? BP::off0(h) / 8 + c : BP::off1(h) / 8 + c - 2;

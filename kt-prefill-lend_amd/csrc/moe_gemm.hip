@@ -649,8 +649,8 @@ __device__ __forceinline__ void gemm_tile(uint8_t* smem, const uint16_t* __restr
       // schedule: the direct loads first, then 32 x (1 MFMA, VPM VALU), an LDS read after
       // every other MFMA and one of the raw weight gathers after every other (each
       // gathers 32 rows' cache lines: in one burst they would hold up the MFMA issue).
-      // VPM covers the type's decode at 256-route tiles (Q4_K and Q8_0 about 2.8 VALU per MFMA,
-      // Q6_K 3.2, IQ3_S 3.5): VALU left over would run after the last MFMA with the matrix
+      // VPM covers the type's decode at 256-route tiles (Q4_K about 2.8 VALU per MFMA, Q8_0 3.2,
+      // IQ3_S 3.5, Q6_K 3.6): VALU left over would run after the last MFMA with the matrix
       // core idle. (128-route tiles have twice that per MFMA; placing 6 to 8 there made no
       // difference.)
       // (gate/up: the direct loads take the first of the per-MFMA VMEM slots instead of a

@@ -621,3 +621,51 @@ def test_window_passes_follow_the_mean(dev, types, T, top_k, hot, mode):
     every token needs several of them."""
     L, _, _ = _pkg()
     _one_popular_slot(dev, types, 256, 256, hot, T, top_k, L.MODE_DECODE if mode == "decode" else L.MODE_GROUPED)
+
+
+@pytest.mark.parametrize("t", [R.GGML_Q8_0, R.GGML_Q6_K])
+@pytest.mark.parametrize("T,mode", [(9, "decode"), (40, "grouped"), (300, "grouped")])
+def test_matrix_decoders_infinite_scale(dev, t, T, mode):
+    """A block whose scale is infinite dequantises to +-inf (the codes' signs), also in the matrix
+    kernels: activations and all other weights positive, so that a down row with such a block
+    gives +-inf, a gate row with one makes its slot's outputs inf, and the rest stays finite."""
+    L, _, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=512, inter=256, hot=3, experts=16, top_k=2, types=(t, t, t))
+    rng = np.random.default_rng(t + T)
+    size, at = (34, 0) if t == R.GGML_Q8_0 else (210, 208)
+
+    def blocks(shape, neg_row=None, inf_at=()):
+        b = np.empty(shape[:2] + (shape[2] // size, size), np.uint8)
+        d = rng.uniform(1e-5, 2e-5, b.shape[:3]).astype(np.float16)
+        for i in inf_at:
+            d[i] = np.inf
+        if t == R.GGML_Q8_0:
+            q = rng.integers(1, 127, b.shape[:3] + (32,))
+            if neg_row is not None:
+                q[:, neg_row] *= -1
+            b[..., 2:] = q.astype(np.int8).view(np.uint8)
+        else:  # codes 33..63, or 1..31 in the negative row
+            b[..., :128] = rng.integers(1, 16, b.shape[:3] + (128,)) | rng.integers(1, 16, b.shape[:3] + (128,)) << 4
+            hi = rng.integers(0, 256, b.shape[:3] + (64,)) & 0x55
+            b[..., 128:192] = hi | 0xAA
+            if neg_row is not None:
+                b[:, neg_row, :, 128:192] = hi[:, neg_row]
+            b[..., 192:208] = rng.integers(1, 128, b.shape[:3] + (16,))
+        b[..., at:at + 2] = d.view(np.uint8).reshape(d.shape + (2,))
+        return b.reshape(shape)
+
+    s13, s2 = (a.shape for a in S.slot_tensors(w))
+    w13 = blocks(s13, inf_at=[(2, 17, 1)])  # gate row 17 of slot 2
+    w2 = blocks(s2, neg_row=9, inf_at=[(0, 9, 0), (1, 40, 0)])
+    slot = np.stack([np.arange(T) % 3, np.full(T, -1)], 1).astype(np.int32)
+    tw = np.full((T, 2), 0.5, np.float32)
+    xb = R.bf16_bits(rng.uniform(0.1, 1.0, (T, w.hidden)).astype(np.float32))
+    got = R.bf16_to_f32(_run(dev, w, xb, tw, slot, w13, w2, L.MODE_DECODE if mode == "decode" else L.MODE_GROUPED))
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    with np.errstate(invalid="ignore"):
+        exp = R.ffn_reference(xb, slot, tw, g, d)
+    inf = np.isinf(exp)
+    assert inf[0::3, 9].all() and inf[1::3, 40].all() and inf[2::3].all() and not inf.all() and not np.isnan(exp).any()
+    assert np.array_equal(got[inf], exp[inf].astype(np.float32))
+    assert R.rel_errors(got[~inf], exp[~inf])[0] < TOL_REL_L2
