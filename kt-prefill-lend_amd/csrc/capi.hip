@@ -270,8 +270,8 @@ int ktmi_moe_layer(const ktmi_layer* L, const void* x, const float* topk_w, cons
   const int64_t K = L->hidden, N = L->inter;
   if (mode == KTMI_MODE_DECODE) {
     KTMI_REQUIRE(decode_mfma_fits(L, tokens, top_k), KTMI_EINVAL,
-                 "moe_layer: the decode mode takes at most %d routes of %d tokens, at most 512 slots, and hidden and "
-                 "intermediate sizes that are multiples of 256",
+                 "moe_layer: the decode mode takes at most %d routes of %d tokens, at most 512 slots, hidden and "
+                 "intermediate sizes that are multiples of 256, and slot matrices under 4 GiB",
                  DM_MAX_ROUTES, DM_MAX_TOKENS);
     return launch_decode_mfma(L, (const uint16_t*)x, topk_w, slot_ids, tokens, top_k, (uint16_t*)y, (uint8_t*)workspace,
                               s);

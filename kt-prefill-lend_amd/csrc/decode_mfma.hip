@@ -574,9 +574,13 @@ int launch_dm_down(const ktmi_layer* L, const uint16_t* hbuf, const int32_t* slo
 
 }  // namespace
 
-// what the kernels take, whatever the mode
+// what the kernels take, whatever the mode; a slot's matrix, x, h and yv are addressed by buffer
+// instructions with 32-bit offsets
 static bool window_shape(const ktmi_layer* L) {
-  return L->hidden % 256 == 0 && L->inter % 256 == 0 && L->n_slots <= 512;
+  const int64_t K = L->hidden, N = L->inter, limit = 0xFFFF0000ll;
+  if (!blck_size(L->type13) || !blck_size(L->type2)) return false;
+  return K % 256 == 0 && N % 256 == 0 && L->n_slots <= 512 && 2 * DM_ROUTES * (K > N ? K : N) <= limit &&
+         2 * N * row_bytes(K, L->type13) <= limit && K * row_bytes(N, L->type2) <= limit;
 }
 
 bool decode_mfma_fits(const ktmi_layer* L, int64_t tokens, int64_t top_k) {

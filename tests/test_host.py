@@ -66,6 +66,25 @@ def test_layer_workspace_sizes():
     assert L.ktmi_moe_layer(d, 0, 0, 0, 1, 8, 0, 0, 0, 0, 0) == -1  # null weights
 
 
+@pytest.mark.parametrize("hidden,inter,t13,t2", [(4096, 524288, 8, 12), (524288, 4096, 12, 8), (1 << 22, 256, 12, 12)])
+def test_decode_mode_slot_matrix_limit(hidden, inter, t13, t2):
+    """The decode-sized kernels address a slot's matrix with 32-bit offsets: one of 4 GiB and more
+    (gate/up, down, or a row of x past the range) takes the GEMV mode, half of it the decode mode."""
+    from kt_prefill_lend_amd import _lib
+
+    L = _lib.lib()
+    p = 1 << 24
+    d = _lib.ktmi_layer(hidden=hidden, inter=inter, n_slots=8, type13=t13, type2=t2, w13=p, w2=p)
+    assert L.ktmi_moe_layer_mode(d, 8, 8) == _lib.MODE_GEMV
+    assert L.ktmi_moe_layer(d, p, p, p, 8, 8, p, p, 1 << 62, _lib.MODE_DECODE, 0) == -1
+    assert b"decode mode" in L.ktmi_last_error()
+    d = _lib.ktmi_layer(hidden=min(hidden, 1 << 19) // (2 if hidden > inter else 1), inter=inter // (2 if inter > hidden else 1),
+                        n_slots=8, type13=t13, type2=t2, w13=p, w2=p)
+    assert L.ktmi_moe_layer_mode(d, 8, 8) == _lib.MODE_DECODE
+    d.type2 = 23  # no kernel: refused by the layer call, no division here
+    assert L.ktmi_moe_layer_mode(d, 8, 8) == _lib.MODE_GEMV
+
+
 @pytest.mark.parametrize("t", TYPES)
 def test_host_quantiser_round_trip(t):
     from kt_prefill_lend_amd import gguf
