@@ -66,7 +66,7 @@ def test_layer_workspace_sizes():
     assert L.ktmi_moe_layer(d, 0, 0, 0, 1, 8, 0, 0, 0, 0, 0) == -1  # null weights
 
 
-@pytest.mark.parametrize("hidden,inter,t13,t2", [(4096, 524288, 8, 12), (524288, 4096, 12, 8), (1 << 22, 256, 12, 12)])
+@pytest.mark.parametrize("hidden,inter,t13,t2", [(4096, 524288, 8, 12), (524288, 8192, 21, 8), (1 << 22, 256, 12, 12)])
 def test_decode_mode_slot_matrix_limit(hidden, inter, t13, t2):
     """The decode-sized kernels address a slot's matrix with 32-bit offsets: one of 4 GiB and more
     (gate/up, down, or a row of x past the range) takes the GEMV mode, half of it the decode mode."""
