@@ -207,3 +207,60 @@ def test_window_ring_drops_the_loads_past_the_last_column(window_kernels):
             if soff != "0":
                 d = _last_def(lines, i, soff)
                 assert re.match(r"s_cselect_b32 s\d+, \S+, 0$", d), (name, "scalar offset of a dropped load", lines[i].strip(), d)
+
+
+def _blocks_of_loop(lines, at):
+    """Line numbers of the innermost loop around line `at`, from the compiler's notes at the blocks
+    (some of a loop's blocks lie behind its end), and the header's."""
+    header, of = {}, None
+    for i, l in enumerate(lines):
+        m = re.match(r"^\.L(BB\w+):|^; %bb", l)
+        if m:
+            note = l + lines[i + 1] + lines[i + 2]
+            inner = re.search(r"in Loop: Header=(BB\w+)", l)
+            of = m.group(1) if "Loop Header" in note.split("\t")[0] and m.group(1) else inner and inner.group(1)
+        header[i] = of
+    assert header[at], "a loop"
+    return [i for i in header if header[i] == header[at]], next(i for i, l in enumerate(lines) if l.startswith(f".L{header[at]}:"))
+
+
+def _entered_at(lines, i):
+    """Where line i's block is entered: i itself, or the branch to it if it lies out of line."""
+    lab = next(j for j in range(i, -1, -1) if lines[j].startswith(".LBB"))
+    m = re.match(r"^\.(LBB\w+):", lines[lab]).group(1)
+    src = [j for j, l in enumerate(lines) if re.search(rf"s_cbranch_execnz \.{m}$", l.split(";")[0].rstrip())]
+    return src[0] if src else i
+
+
+def test_window_ring_counted_wait_covers_the_next_column(window_kernels):
+    for name, lines in window_kernels.items():
+        mark = [i for i, l in enumerate(lines) if "sched_barrier mask(0x00000000)" in l]
+        assert len(mark) == 1, (name, "one scheduling barrier, ahead of the counted wait", mark)
+        loop, head = _blocks_of_loop(lines, mark[0])
+        wait = next(i for i in loop if i > mark[0] and "s_waitcnt" in lines[i] and "vmcnt" in lines[i])
+        n = _vmcnt(lines[wait])
+        dma = [i for i in loop if DMA.match(lines[i])]
+        entered = [_entered_at(lines, i) for i in dma]
+        assert dma and min(entered) > wait, (name, "direct loads before the wait")
+        # this column's activation loads, but for those that a branch jumps over
+        skipped = _skipped(lines, head, mark[0])
+        x = [i for i in loop if head < i < mark[0] and VMEM.match(lines[i]) and i not in skipped]
+        assert 0 < n <= len(dma) + len(x), (name, n, len(dma), len(x))
+        # the prologue holds both columns' direct loads
+        pro = [i for i, l in enumerate(lines) if DMA.match(l) and i not in dma]
+        assert len(pro) >= 2 * len(dma), (name, "prologue", len(pro), len(dma))
+        # read out before the buffer is loaded again
+        reads = [i for i in range(wait, min(entered)) if re.match(r"^\s*ds_read", lines[i])]
+        done = [i for i in range(wait, min(entered)) if re.search(r"s_waitcnt.*lgkmcnt\(0\)", lines[i])]
+        assert reads and done and max(reads) < max(done), (name, "LDS reads of the column")
+
+
+def _skipped(lines, a, b):
+    """Lines of [a, b) that a forward branch in it to a label up to b jumps over."""
+    label = {m.group(1): i for i in range(a, b + 1) if (m := re.match(r"^(\.LBB\w+):", lines[i]))}
+    out = set()
+    for i in range(a, b):
+        m = re.search(r"s_c?branch\w*\s+(\.LBB\w+)", lines[i])
+        if m and label.get(m.group(1), -1) > i and "execz" not in lines[i]:
+            out.update(range(i + 1, label[m.group(1)]))
+    return out
