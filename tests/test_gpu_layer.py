@@ -669,3 +669,81 @@ def test_matrix_decoders_infinite_scale(dev, t, T, mode):
     assert inf[0::3, 9].all() and inf[1::3, 40].all() and inf[2::3].all() and not inf.all() and not np.isnan(exp).any()
     assert np.array_equal(got[inf], exp[inf].astype(np.float32))
     assert R.rel_errors(got[~inf], exp[~inf])[0] < TOL_REL_L2
+
+
+def _random_weights(rng, t, shape):
+    """Slot weights of random codes with finite scales of both signs, sized as quantised ~N(0, 0.02)
+    weights."""
+    size, at, mag = {R.GGML_Q8_0: (34, (0,), 3e-4), R.GGML_Q4_K: (144, (0, 2), 1e-4), R.GGML_Q6_K: (210, (208,), 2e-5),
+                     R.GGML_IQ3_S: (110, (0,), 2e-4)}[t]
+    b = rng.integers(0, 256, size=shape, dtype=np.uint8).reshape(-1, size)
+    for o in at:
+        d = (rng.uniform(0.5, 1.0, b.shape[0]) * mag * rng.choice([-1.0, 1.0], b.shape[0])).astype(np.float16)
+        b[:, o:o + 2] = d.view(np.uint8).reshape(-1, 2)
+    return b.reshape(shape)
+
+
+@pytest.mark.parametrize("types", [(R.GGML_Q8_0, R.GGML_Q8_0), (R.GGML_Q4_K, R.GGML_Q6_K), (R.GGML_Q6_K, R.GGML_Q4_K),
+                                   (R.GGML_IQ3_S, R.GGML_IQ3_S)])
+@pytest.mark.parametrize("hidden,inter", [(4096, 1024), (7168, 512)])
+@pytest.mark.parametrize("T,top_k", [(9, 2), (30, 3), (50, 4), (38, 8)])
+def test_window_long_rows(dev, types, hidden, inter, T, top_k):
+    """The decode-sized kernels where a wave takes 4 and 7 columns of a gate/up row and 2 and 4 of a
+    down row, so that both buffers of its ring are filled again: passes of 16, 32 and 64 routes,
+    up to 256 routes and (but for Q6_K gate/up, which the grouped mode's GEMMs take) past them,
+    twice with the same bits; against the fp64 FFN."""
+    L, _, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=hidden, inter=inter, hot=3, experts=16, top_k=top_k, types=(types[0], types[0], types[1]))
+    rng = np.random.default_rng(types[0] + hidden + T)
+    slot = rng.integers(-1, w.hot, size=(T, top_k)).astype(np.int32)
+    slot[:, 0] = 1
+    tw = rng.random((T, top_k)).astype(np.float32)
+    tw /= tw.sum(axis=1, keepdims=True)
+    xb = S.activations(w, T)
+    w13 = _random_weights(rng, types[0], (w.hot, 2 * inter, R.row_bytes(hidden, types[0])))
+    w2 = _random_weights(rng, types[1], (w.hot, hidden, R.row_bytes(inter, types[1])))
+    mode = L.MODE_DECODE if T * top_k <= 256 else L.MODE_GROUPED
+    y = _run(dev, w, xb, tw, slot, w13, w2, mode)
+    assert np.array_equal(y, _run(dev, w, xb, tw, slot, w13, w2, mode))
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    l2, l1, cos = R.rel_errors(R.bf16_to_f32(y), R.ffn_reference(xb, slot, tw, g, d))
+    assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0].split("-")[0] for c in CASES])
+def test_gemms_vs_ffn_reference(dev, case):
+    """The layer reference test on the sort, the GEMMs and their combine (160 tokens: past the
+    chunks that the grouped mode gives to the decode-sized kernels)."""
+    test_layer_vs_ffn_reference(dev, (case[0], 160) + tuple(case[2:]), "grouped")
+
+
+def test_slot_address_table_128_route_tiles(dev):
+    """Slot address tables against contiguous slots in the GEMMs of 128-route tiles."""
+    test_slot_address_table_matches_contiguous_slots(dev, "grouped", 300)
+
+
+@pytest.mark.parametrize("top_k", [1, 5])
+def test_gemm_edge_cases(dev, top_k):
+    """The sort, the GEMMs and their combine on an empty slot, a slot of one route, tokens without a
+    hot route (exactly zero) and slot ids of no slot here (the same bits as -1); against the fp64 FFN."""
+    L, _, S = _pkg()
+    base = S.WORKLOADS["q4_k+q6_k-h2048-n512-e256-k8-hot40-prefill"]
+    w = replace(base, hidden=512, inter=256, hot=8, experts=32, top_k=top_k)
+    T = 150
+    rng = np.random.default_rng(41 + top_k)
+    slot = rng.integers(-1, 5, size=(T, top_k)).astype(np.int32)  # slots 5 and 6 empty
+    slot[:10] = -1
+    slot[77, 0] = 7
+    tw = rng.random((T, top_k)).astype(np.float32)
+    xb = S.activations(w, T)
+    w13, w2 = S.slot_tensors(w)
+    y = _run(dev, w, xb, tw, slot, w13, w2, L.MODE_GROUPED)
+    foreign = np.where(slot < 0, rng.choice([-7, w.hot, w.hot + 5], size=slot.shape), slot).astype(np.int32)
+    assert np.array_equal(y, _run(dev, w, xb, tw, foreign, w13, w2, L.MODE_GROUPED))
+    got = R.bf16_to_f32(y)
+    cold = (slot < 0).all(axis=1)
+    assert cold[:10].all() and np.all(got[cold] == 0)
+    g, d = dequant_w(w13, w2, w.types, w.hidden, w.inter)
+    l2, l1, cos = R.rel_errors(got[~cold], R.ffn_reference(xb, slot, tw, g, d)[~cold])
+    assert l2 < TOL_REL_L2 and cos > 0.999, (l2, l1, cos)

@@ -66,6 +66,28 @@ def test_layer_workspace_sizes():
     assert L.ktmi_moe_layer(d, 0, 0, 0, 1, 8, 0, 0, 0, 0, 0) == -1  # null weights
 
 
+def test_auto_mode_on_long_rows():
+    """Below 64 routes AUTO takes the GEMV mode where its two launches fit and the decode mode
+    where the rows are too long for them (more than 64 weight units gate/up or 16 down), within the
+    decode mode's own limits."""
+    from kt_prefill_lend_amd import _lib
+
+    L = _lib.lib()
+
+    def mode(tokens, top_k, hidden, inter, t13=12, t2=14, slots=24):
+        d = _lib.ktmi_layer(hidden=hidden, inter=inter, n_slots=slots, type13=t13, type2=t2)
+        return L.ktmi_moe_layer_mode(d, tokens, top_k)
+
+    assert mode(4, 8, 2048, 512) == _lib.MODE_GEMV and mode(8, 8, 2048, 512) == _lib.MODE_DECODE
+    assert mode(1, 1, 7168, 2048) == mode(5, 8, 7168, 2048) == _lib.MODE_DECODE
+    assert mode(4, 8, 2048, 512, 8, 8) == _lib.MODE_GEMV and mode(4, 8, 2048, 768, 8, 8) == _lib.MODE_DECODE
+    assert mode(4, 8, 4096, 1024) == _lib.MODE_GEMV and mode(4, 8, 4352, 1024) == _lib.MODE_DECODE
+    assert mode(5, 8, 7168, 2048, slots=513) == _lib.MODE_GEMV  # past the decode mode's slots
+    assert mode(65, 3, 7168, 2048) == _lib.MODE_GEMV            # and its tokens
+    assert mode(5, 8, 7168, 2016, 12, 8) == _lib.MODE_GEMV      # and its multiples of 256
+    assert mode(33, 8, 7168, 2048) == _lib.MODE_GROUPED
+
+
 @pytest.mark.parametrize("hidden,inter,t13,t2", [(4096, 524288, 8, 12), (524288, 8192, 21, 8), (1 << 22, 256, 12, 12)])
 def test_decode_mode_slot_matrix_limit(hidden, inter, t13, t2):
     """The decode-sized kernels address a slot's matrix with 32-bit offsets: one of 4 GiB and more
