@@ -540,6 +540,9 @@ int launch_dm_gate_up(const ktmi_layer* L, const uint16_t* x, const int32_t* slo
   const int64_t m = pass_routes(tokens, R, S);
   if (R <= 256) {
     if (m <= 16) KTMI_GU(1, 4); else if (m <= 32) KTMI_GU(2, 4); else KTMI_GU(4, 4);
+  } else if constexpr (TYPE == GGML_Q6_K) {
+    set_error("window gate/up: %lld routes of Q6_K (window_fits leaves them to the GEMMs)", (long long)R);
+    return KTMI_EINVAL;
   } else {
     if (m <= 32) KTMI_GU(2, 16); else KTMI_GU(4, 16);
   }
