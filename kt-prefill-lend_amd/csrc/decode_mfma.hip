@@ -238,6 +238,11 @@ struct ColRing {
 // both halves), its weight bytes out of LDS into registers, the direct loads of column
 // sb + NB into the buffer just read, then (G > 1) the activation loads of the second half; the
 // decode of a half (about 450 VALU cycles a tile) runs while its activation loads are in flight.
+// Loads return in order, so at G > 1 the wait for the second half's activations also completes
+// the direct loads before them: the ring then covers a half of a column's work, not a column. At
+// G = 1 the next columns' loads stay in flight for Q4_K and Q8_0; the direct loads of Q6_K and
+// IQ3_S are under lane masks (padding chunks), where the compiler counts none of them and its
+// waits for the activations drain the ring too.
 template <int TYPE, int NT, int NB, int G>
 __device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring, const __amdgpu_buffer_rsrc_t& act,
                                                const uint32_t (&xoff)[G], int ng, int sb0, int sb1,
@@ -265,7 +270,8 @@ __device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring
     if constexpr (G == 1) xissue(sb, H1{});
     __builtin_amdgcn_sched_barrier(0);  // the activation loads stay ahead of the wait that counts them
     // the column's direct loads have landed once at most the younger operations are in flight:
-    // the next column's (NB = 2) and this column's activation loads (at least 4, 8 at G = 1)
+    // the next column's (NB = 2) and this column's activation loads (at least 4, 8 at G = 1); the
+    // numbers are checked against the compiled code by a test
     constexpr int NX = G == 1 ? 8 : 4;
     __builtin_amdgcn_s_waitcnt(dm_vmcnt((NB - 1) * ColRing<TYPE, NT, NB>::NI + NX));
     wave_fence();
@@ -317,7 +323,8 @@ __device__ __forceinline__ int2 block_slot(const int32_t* __restrict__ slot_ids,
   return make_int2(e, slot_routes(wr, e, mem));
 }
 
-// waves a SIMD the registers leave room for without spilling
+// waves a SIMD that the registers are held to, without spilling but for Q6_K at G = 4 (13). For
+// Q8_0 at G = 1 the rings (70 KB a block) leave two blocks a CU whatever it says
 template <int TYPE, int G>
 constexpr int dm_waves() {
   return G == 4 ? 2 : G == 1 ? (TYPE == GGML_Q4_K ? 4 : 3) : TYPE == GGML_Q4_K || TYPE == GGML_Q8_0 ? 3 : 2;
@@ -411,7 +418,8 @@ __global__ __launch_bounds__(DM_THREADS, (dm_waves<TYPE, G>())) void dm_gate_up(
 // to bf16 (the reference's per-route bf16 output), to yv [R, K]. The weighted top-k sum is a
 // launch of its own (dm_combine): inside this one, the blocks of a tile would have to order
 // themselves through device-scope fences, which write back and invalidate the whole L2 of
-// their XCD.
+// their XCD. The registers are held to 4, 3 and 2 waves a SIMD; Q6_K at NT = 2, G = 4 spills 9 of
+// them for it and IQ3_S at NT = 2, G = 2 three.
 template <int TYPE, int NT, int G, int NR, int NB>
 __global__ __launch_bounds__(DM_THREADS, (G == 1 ? 4 : G == 2 ? 3 : 2)) void dm_down(const uint16_t* __restrict__ hbuf, int K, int N,
                                                       const int32_t* __restrict__ slot_ids, int R, int S,

@@ -22,7 +22,9 @@ namespace ktmi {
 // memory order: every store instruction writes whole 256-byte segments. With a lane to a row
 // and the chunks stored straight from the registers, an instruction touched 64 segments and
 // eight 7168 x 2048 Q6_K experts took 144 us (2.3 TB/s); so they take 67 us (4.9 TB/s,
-// the rate of a large copy on this card).
+// the rate of a large copy on this card). The stores are non-temporal: 43 against 54 us for
+// eight such Q4_K experts, and no slower for a reader that follows, down to one expert of 1024 x
+// 2048 (with a pass over the output behind it 11.4 us either way).
 constexpr int DQ_UNITS = 16;                      // (row, column) units a wave
 constexpr int DQ_STG = DQ_UNITS * 256;            // staging bytes a wave: 128 bf16 values a unit
 
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
   BP::load_head(row, sb, h, hd);
   if (inside(BP::template ksub_hp<0>(p))) BP::template load_hp<0>(row, sb, h, p, grid, rw[0]);
   if (inside(BP::template ksub_hp<1>(p))) BP::template load_hp<1>(row, sb, h, p, grid, rw[1]);
-  __builtin_amdgcn_sched_barrier(0);  // (67 us without it)
+  __builtin_amdgcn_sched_barrier(0);  // the same eight experts back to back: 62 us, 65 without it
   uint8_t* stg = stage + wave * DQ_STG;
   uint16_t* oe = out + e * out_stride;
   auto half = [&](auto s2c) {
