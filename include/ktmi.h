@@ -116,7 +116,7 @@ int ktmi_combine(const void* out, int dtype, const float* w, int64_t T, int64_t 
  * routes (< 0, the CPU's) contribute nothing. Deterministic (no atomics on outputs).
  * w13: slot tensor uint8 [n_slots, 2*inter, row_bytes(hidden, type13)], rows [gate; up];
  * w2: uint8 [n_slots, hidden, row_bytes(inter, type2)]; with w_is_table = 1 both are int64
- * device tables of per-slot addresses. x, y bf16 [tokens, hidden]; topk_w fp32.
+ * device tables of per-slot addresses (16-byte aligned, as a slot tensor's are). x, y bf16 [tokens, hidden]; topk_w fp32.
  * Replaces KTGGUFHotExpertsMethod.apply (hot/kt_gguf_hot.py:240-304) and the streamer's
  * per-group dequant + cutlass_fused_moe body (P:40789-40819). */
 typedef struct ktmi_layer {
@@ -137,7 +137,7 @@ int ktmi_moe_layer(const ktmi_layer* layer, const void* x, const float* topk_w, 
                    void* stream);
 /* The mode KTMI_MODE_AUTO picks for this many routes: GROUPED above 256 routes, DECODE from
  * 64 routes where it applies (and below where the sizes are past the GEMV mode's fused
- * launches), else GEMV. */
+ * launches; not on long Q8_0 rows with about a route a slot or less), else GEMV. */
 int ktmi_moe_layer_mode(const ktmi_layer* layer, int64_t tokens, int64_t top_k);
 /* Tokens per pass of KTMI_MODE_GROUPED: a longer call runs as consecutive passes over token
  * slices of this size (each token's output depends only on its own routes), and the

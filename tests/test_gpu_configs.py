@@ -74,8 +74,7 @@ def test_q4_k_decode_windows(dev, T, mode):
 @pytest.mark.parametrize("T", [8, 16, 25])
 def test_iq3_s_decode_mode_windows(dev, T):
     """The decode mode on the IQ3_S workload at its real shape (hidden 2048, top-10: 80 / 160 /
-    250 routes), where its staged rows fit; the Q8_0 and Q6_K rows of hidden 2048 do not
-    (decode_mfma_fits) and those layers take the GEMV mode."""
+    250 routes)."""
     L, _, _ = _pkg()
     _check(dev, "iq3_s-h2048-n512-e512-k10-hot48", T, L.MODE_DECODE, 1)
 
