@@ -189,16 +189,20 @@ static int scratch_of_current_device(void** out) {
 // 64, 38.4 / 25.8 at 128; Q8_0 29.8 / 29.0, 39.2 / 34.7).
 // Where the rows are too long for those two launches, the decode mode starts at one route: its
 // alternative is the stage-by-stage GEMV (7168 x 2048 Q4_K/Q6_K, 7 tokens: 164 against 60 us).
-// Above one or two routes a slot the decode mode is also the faster one on long rows of Q8_0 (2048 x
-// 512, 32 slots: the line above); with hardly one, both are bound by the weights' bytes, which the
-// GEMV's loads bring at 6.9 TB/s and the decode mode's ring at 5.3 (128 slots all hot, 16 tokens: 62
-// against 75 us). The decode mode stays there for its smaller error (0.005 against 0.0125).
+// With hardly a route a slot on long rows of Q8_0 both are bound by the weights' bytes, which the
+// GEMV's loads bring at 6.9 TB/s and the decode mode's ring at 5.3: there the GEMV stays (2048 x 512,
+// 128 slots all hot, 16 tokens 62 against 75 us; 256 slots, 32 tokens 104 against 147; 1024 rows of
+// Q4_K down, 128 slots, 24 tokens 118 against 148), up to a mean of one route a slot at 512 rows:
+// past it the gain is within the 10 % that the decode mode's smaller error is worth.
 constexpr int64_t kDecodeMinRoutes = 64;
 
 int ktmi_moe_layer_mode(const ktmi_layer* L, int64_t tokens, int64_t top_k) {
   if (tokens * top_k > kGemvMaxRoutes) return KTMI_MODE_GROUPED;
   if (!L || !decode_mfma_fits(L, tokens, top_k)) return KTMI_MODE_GEMV;
-  return tokens * top_k >= kDecodeMinRoutes || !decode_layer_fits(L, tokens, top_k) ? KTMI_MODE_DECODE : KTMI_MODE_GEMV;
+  if (!decode_layer_fits(L, tokens, top_k)) return KTMI_MODE_DECODE;
+  const int64_t R = tokens * top_k;
+  const bool few = L->type13 == GGML_Q8_0 && L->hidden > 1024 && 512 * R <= L->inter * L->n_slots;
+  return R >= kDecodeMinRoutes && !few ? KTMI_MODE_DECODE : KTMI_MODE_GEMV;
 }
 
 static int64_t gemv_layer_workspace(const ktmi_layer* L, int64_t tokens, int64_t top_k) {

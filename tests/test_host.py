@@ -88,6 +88,24 @@ def test_auto_mode_on_long_rows():
     assert mode(33, 8, 7168, 2048) == _lib.MODE_GROUPED
 
 
+def test_auto_mode_with_hardly_a_route_a_slot():
+    """Long rows of Q8_0 with at most one route a slot on average (at 512 intermediate rows) stay
+    with the GEMV mode past 64 routes; other types, more routes and short rows take the decode mode."""
+    from kt_prefill_lend_amd import _lib
+
+    L = _lib.lib()
+
+    def mode(tokens, slots, hidden=2048, inter=512, t13=8, t2=8):
+        d = _lib.ktmi_layer(hidden=hidden, inter=inter, n_slots=slots, type13=t13, type2=t2)
+        return L.ktmi_moe_layer_mode(d, tokens, 8)
+
+    assert mode(8, 64) == mode(16, 128) == mode(32, 256) == _lib.MODE_GEMV
+    assert mode(8, 63) == mode(17, 128) == mode(31, 247) == _lib.MODE_DECODE
+    assert mode(16, 64, inter=1024, t2=12) == _lib.MODE_GEMV and mode(17, 64, inter=1024, t2=12) == _lib.MODE_DECODE
+    assert mode(8, 128, t13=12, t2=12) == mode(8, 128, t13=21, t2=21) == mode(8, 128, hidden=1024) == _lib.MODE_DECODE
+    assert mode(8, 128, inter=768) == _lib.MODE_DECODE  # a down row past the GEMV mode's 16 units
+
+
 @pytest.mark.parametrize("hidden,inter,t13,t2", [(4096, 524288, 8, 12), (524288, 8192, 21, 8), (1 << 22, 256, 12, 12)])
 def test_decode_mode_slot_matrix_limit(hidden, inter, t13, t2):
     """The decode-sized kernels address a slot's matrix with 32-bit offsets: one of 4 GiB and more
