@@ -24,8 +24,10 @@
 //   Q8_0, IQ3_S: positions [32h, 32h+32) (one Q8_0 block, one IQ3_S 32-group)
 // `off0`/`off1` give the step positions of out[0..7] and out[8..15] (16 values each).
 //
-// Zero codes and infinite or negative scales give what a plain product gives (d * -0, +-inf), in
-// every kernel: the dequant entry point, whose bytes are its result, runs the same bodies.
+// Infinite scales give what a plain product gives (+-inf) in every kernel; so do zero codes (d * -0)
+// in the GEMMs and in the dequant entry point, whose bytes are its result and which runs the same
+// bodies. Where a kernel takes the other form (decode_hp<S2, PLAIN = false>) a zero's sign may
+// differ, which no sum of products sees.
 //
 // Every SUB-dependent member also exists with the step parity as a run-time value: the
 // `_hp<S2>(..., p)` forms take SUB = 2 S2 + p with S2 a compile-time constant and p a
@@ -86,8 +88,7 @@ __device__ __forceinline__ float fma_code(float d, uint32_t w, float c) {
   return __builtin_fmaf(d, (float)q, c);
 }
 // unsigned codes less MID in both half-words of w, as signed fp16 denormals: one v_pk_add_f16,
-// exact. Taking MID d from the FMA instead would spare it (7168 x 2048 Q8_0, 5 tokens 147 against
-// 150 us, most layers within 1 %), but give inf - inf where d is infinite and +0 for every zero
+// exact
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 template <int MID>
 __device__ __forceinline__ uint32_t code_sub(uint32_t w) {
@@ -105,6 +106,17 @@ __device__ __forceinline__ float minus_zero() {
 __device__ __forceinline__ void codes4(float d, float c, uint32_t e, uint32_t o, uint32_t* out) {
   out[0] = f2bf2(fma_code<0>(d, e, c), fma_code<0>(d, o, c));
   out[1] = f2bf2(fma_code<1>(d, e, c), fma_code<1>(d, o, c));
+}
+
+// the same of codes that hold q + MID: the plain product (PLAIN; d * -0 and +-inf as they are) or,
+// for finite d only, its value by taking MID d from the FMA (+0 for every zero; inf - inf where d is
+// infinite), 2 of 11 VALU less. The GEMMs, within 1 % of the same time either way, and the dequant
+// entry point take the first, the decode-sized kernels the second where `unbounded` finds no
+// infinite or NaN scale
+template <int MID, bool PLAIN>
+__device__ __forceinline__ void biased4(float d, float c, uint32_t e, uint32_t o, uint32_t* out) {
+  if constexpr (PLAIN) codes4(d, minus_zero(), code_sub<MID>(e), code_sub<MID>(o), out);
+  else codes4(d, c, e, o, out);
 }
 
 // Where a piece's bytes are read from: global memory (through the caches) or LDS (rows a
@@ -216,7 +228,8 @@ struct BPiece<GGML_Q4_K> : NoLookup<BPiece<GGML_Q4_K>> {
   __device__ __forceinline__ static void load_hp(const uint8_t* row, int sb, int h, int p, const uint32_t*, Raw& r) {
     r.q = M::template ld<u32x4_t>(row + sb * QB4_K + 16 + 64 * S2 + 32 * p + 16 * h);
   }
-  template <int S2>
+  __device__ static bool unbounded(const Head&, const Raw&) { return false; }
+  template <int S2, bool PLAIN = true>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t*, int p,
                                                    uint32_t out[16]) {
     const float d = half_bits_to_float(hd.hdr[0] & 0xFFFF);
@@ -277,7 +290,10 @@ struct BPiece<GGML_Q8_0> : NoLookup<BPiece<GGML_Q8_0>> {
     }
     r.w[8] = M::template ld<uint32_t>(a + 8);
   }
-  template <int S2>
+  __device__ static bool unbounded(const Head&, const Raw& r) {
+    return ((r.s ? r.w[0] >> 16 : r.w[0]) & 0x7C00u) == 0x7C00u;
+  }
+  template <int S2, bool PLAIN = true>
   __device__ __forceinline__ static void decode_hp(const Head&, const Raw& r, const uint32_t*, int, uint32_t out[16]) {
     const float d = half_bits_to_float((uint16_t)(r.s ? r.w[0] >> 16 : r.w[0] & 0xFFFFu));
     // the block's codes start 2 bytes past its d: bytes 0 and 2 of word i are bytes 2 and 4
@@ -287,7 +303,7 @@ struct BPiece<GGML_Q8_0> : NoLookup<BPiece<GGML_Q8_0>> {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t lo = r.w[i] ^ 0x80808080u, hi = r.w[i + 1] ^ 0x80808080u;
-      codes4(dn, minus_zero(), code_sub<128>(__builtin_amdgcn_perm(hi, lo, even)), code_sub<128>(__builtin_amdgcn_perm(hi, lo, odd)), out + 2 * i);
+      biased4<128, PLAIN>(dn, -128.0f * d, __builtin_amdgcn_perm(hi, lo, even), __builtin_amdgcn_perm(hi, lo, odd), out + 2 * i);
     }
   }
   __device__ static int off0(int h) { return 32 * h; }
@@ -334,7 +350,8 @@ struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
       for (int i = 0; i < 4; ++i) r.qh[i] = prev.qh[i];
     }
   }
-  template <int S2>
+  __device__ static bool unbounded(const Head& hd, const Raw&) { return (hd.d & 0x7C00u) == 0x7C00u; }
+  template <int S2, bool PLAIN = true>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t*, int p,
                                                    uint32_t out[16]) {
     constexpr int hh = S2;
@@ -353,8 +370,8 @@ struct BPiece<GGML_Q6_K> : NoLookup<BPiece<GGML_Q6_K>> {
       const uint32_t lw = r.ql[i], hw = r.qh[i];
       // bits 6 and 7 of the bytes are others' and masked off with the split into half-words
       const uint32_t va = bfi(0x0F0F0F0Fu, lw, hw << (4 - hsh)), vb = bfi(0x0F0F0F0Fu, lw >> 4, hw >> hsh);
-      codes4(fa * kCodeScale, minus_zero(), code_sub<32>(and_opaque(va, 0x003F003Fu)), code_sub<32>(and_opaque(va >> 8, 0x003F003Fu)), out + 2 * i);
-      codes4(fb * kCodeScale, minus_zero(), code_sub<32>(and_opaque(vb, 0x003F003Fu)), code_sub<32>(and_opaque(vb >> 8, 0x003F003Fu)), out + 8 + 2 * i);
+      biased4<32, PLAIN>(fa * kCodeScale, -32.0f * fa, and_opaque(va, 0x003F003Fu), and_opaque(va >> 8, 0x003F003Fu), out + 2 * i);
+      biased4<32, PLAIN>(fb * kCodeScale, -32.0f * fb, and_opaque(vb, 0x003F003Fu), and_opaque(vb >> 8, 0x003F003Fu), out + 8 + 2 * i);
     }
   }
   __device__ static int off0(int h) { return 16 * h; }
@@ -453,7 +470,8 @@ struct BPiece<GGML_IQ3_S> {
       out[2 * k + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u) ^ pair_signs(2 * k + 1);
     }
   }
-  template <int S2>
+  __device__ static bool unbounded(const Head&, const Raw&) { return false; }
+  template <int S2, bool PLAIN = true>
   __device__ __forceinline__ static void decode_hp(const Head& hd, const Raw& r, const uint32_t* grid, int p,
                                                    uint32_t out[16]) {
     Look lk;

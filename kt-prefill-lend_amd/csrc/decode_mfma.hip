@@ -238,13 +238,15 @@ struct ColRing {
 // both halves), its weight bytes out of LDS into registers, the direct loads of column
 // sb + NB into the buffer just read, then (G > 1) the activation loads of the second half; the
 // decode of a half (about 450 VALU cycles a tile) runs while its activation loads are in flight.
+// PLAIN: the decoders' plain products; without it, whether a scale is infinite or NaN, so that the
+// wave has to run the columns again with it.
 // Loads return in order, so at G > 1 the wait for the second half's activations also completes
 // the direct loads before them: the ring then covers a half of a column's work, not a column. At
 // G = 1 the next columns' loads stay in flight for Q4_K and Q8_0; the direct loads of Q6_K and
 // IQ3_S are under lane masks (padding chunks), where the compiler counts none of them and its
 // waits for the activations drain the ring too.
-template <int TYPE, int NT, int NB, int G>
-__device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring, const __amdgpu_buffer_rsrc_t& act,
+template <int TYPE, int NT, int NB, int G, bool PLAIN>
+__device__ __forceinline__ bool window_pass(const ColRing<TYPE, NT, NB>& ring, const __amdgpu_buffer_rsrc_t& act,
                                                const uint32_t (&xoff)[G], int ng, int sb0, int sb1,
                                                const uint32_t* grid, f32x4_t (&acc)[NT][G]) {
   using BP = BPiece<TYPE>;
@@ -265,6 +267,7 @@ __device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring
   using H0 = std::integral_constant<int, 0>;
   using H1 = std::integral_constant<int, 1>;
   int buf = 0;
+  bool rare = false;
   for (int sb = sb0; sb < sb1; ++sb) {
     xissue(sb, H0{});
     if constexpr (G == 1) xissue(sb, H1{});
@@ -291,7 +294,7 @@ __device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring
       constexpr int S2 = decltype(s2c)::value;
       uint32_t a[NT][16];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) BP::template decode_hp<S2>(hd[t], raw[t][S2], grid, p, a[t]);
+      for (int t = 0; t < NT; ++t) BP::template decode_hp<S2, PLAIN>(hd[t], raw[t][S2], grid, p, a[t]);
 #pragma unroll
       for (int cg = 0; cg < G; ++cg)
         if (cg < ng)  // uniform
@@ -301,12 +304,40 @@ __device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring
             for (int t = 0; t < NT; ++t)
               acc[t][cg] = mfma16(words8(&a[t][4 * j]), xv[G == 1 ? S2 : 0][cg][j], acc[t][cg]);
     };
+    if constexpr (!PLAIN)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) rare |= BP::unbounded(hd[t], raw[t][0]) | BP::unbounded(hd[t], raw[t][1]);
     half(H0{});
     if constexpr (G > 1) xissue(sb, H1{});
     half(H1{});
     buf = NB == 2 ? buf ^ 1 : 0;
   }
   __builtin_amdgcn_s_waitcnt(dm_vmcnt(0));  // the loads past the last column have written their zeros
+  return rare;
+}
+
+// The ring's first columns issued, the columns run (acc from zero), and run again with plain
+// products where a scale is infinite: in the loop those cost Q8_0 windows 3 to 4 % (2048 x 512, 16
+// tokens 34.3 us, so 33.1; 7168 x 2048, 5 tokens 152 and 148), and only infinities need them.
+template <int TYPE, int NT, int NB, int G>
+__device__ __forceinline__ void window_columns(const ColRing<TYPE, NT, NB>& ring, const __amdgpu_buffer_rsrc_t& act,
+                                               const uint32_t (&xoff)[G], int ng, int sb0, int sb1,
+                                               const uint32_t* grid, f32x4_t (&acc)[NT][G]) {
+  auto start = [&]() {
+    ring.issue(sb0, 0, sb0 < sb1);
+    if (NB == 2) ring.issue(sb0 + 1, 1, sb0 + 1 < sb1);
+#pragma unroll
+    for (int cg = 0; cg < G; ++cg)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t][cg] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  start();
+  const bool rare = window_pass<TYPE, NT, NB, G, false>(ring, act, xoff, ng, sb0, sb1, grid, acc);
+  if constexpr (TYPE == GGML_Q8_0 || TYPE == GGML_Q6_K)
+    if (__builtin_expect(__any(rare), 0)) {
+      start();
+      window_pass<TYPE, NT, NB, G, true>(ring, act, xoff, ng, sb0, sb1, grid, acc);
+    }
 }
 
 // The k-th slot with routes of this block, its routes listed in mem: (slot, route count), slot
@@ -379,11 +410,7 @@ __global__ __launch_bounds__(DM_THREADS, (dm_waves<TYPE, G>())) void dm_gate_up(
       xoff[cg] = col < m ? (uint32_t)(mem[col] / top_k) * (uint32_t)K * 2u : x_bytes;
     }
     if (cg0 > 0) __syncthreads();  // the previous pass has read the partial sums
-    ring.issue(sb0, 0, sb0 < sb1);
-    if (NB == 2) ring.issue(sb0 + 1, 1, sb0 + 1 < sb1);
     f32x4_t acc[2][G];
-#pragma unroll
-    for (int cg = 0; cg < G; ++cg) acc[0][cg] = acc[1][cg] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     window_columns<TYPE, 2, NB, G>(ring, x_rsrc, xoff, ng, sb0, sb1, grid, acc);
     __syncthreads();  // every wave has read its ring
 #pragma unroll
@@ -461,13 +488,7 @@ __global__ __launch_bounds__(DM_THREADS, (G == 1 ? 4 : G == 2 ? 3 : 2)) void dm_
       const int col = 16 * (cg0 + cg) + r;
       hoff[cg] = col < m ? (uint32_t)mem[col] * hrow : h_bytes;
     }
-    ring.issue(0, 0, true);
-    if (NB == 2) ring.issue(1, 1, nsb > 1);
     f32x4_t acc[NT][G];
-#pragma unroll
-    for (int cg = 0; cg < G; ++cg)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t][cg] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     window_columns<TYPE, NT, NB, G>(ring, h_rsrc, hoff, ng, 0, nsb, grid, acc);
     // lane l holds rows 4 (l / 16) + i of column l % 16: four consecutive bf16 of yv
 #pragma unroll

@@ -624,7 +624,7 @@ def test_window_passes_follow_the_mean(dev, types, T, top_k, hot, mode):
 
 
 @pytest.mark.parametrize("t", [R.GGML_Q8_0, R.GGML_Q6_K])
-@pytest.mark.parametrize("T,mode", [(9, "decode"), (40, "grouped"), (300, "grouped")])
+@pytest.mark.parametrize("T,mode", [(9, "decode"), (30, "decode"), (60, "decode"), (40, "grouped"), (300, "grouped")])
 def test_matrix_decoders_infinite_scale(dev, t, T, mode):
     """A block whose scale is infinite dequantises to +-inf (the codes' signs), also in the matrix
     kernels: activations and all other weights positive, so that a down row with such a block
