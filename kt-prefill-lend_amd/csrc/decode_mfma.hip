@@ -18,8 +18,8 @@
 // What bounds them: the touched weights' bytes (up to 5 TB/s on large experts) and, close
 // behind, the decode (2.5 to 4 VALU a value); on small layers the three launches. The weights
 // pass through LDS one super-block column at a time, so any row length runs at the same
-// occupancy: the 7168 x 2048 Q4_K/Q6_K layer with 24 slots at 5 tokens takes 87 us (stage-by-
-// stage GEMV 189-244), the 2048 x 768 Q8_0 layer with 16 slots at 24 tokens 34 us (168-174).
+// occupancy: the 7168 x 2048 Q4_K/Q6_K layer with 24 slots at 5 tokens takes 92 us (stage-by-
+// stage GEMV 206), the 2048 x 768 Q8_0 layer with 16 slots at 24 tokens 35 us (170).
 //
 // Lane map (16x16x32 operands): row or column l % 16, k-chunk g = l / 16 (8 values). Lane
 // group g holds the piece of BPiece step SUB = 2 s + (g & 1), half g >> 1 of each 128-value
@@ -354,7 +354,7 @@ __device__ __forceinline__ int2 block_slot(const int32_t* __restrict__ slot_ids,
   return make_int2(e, slot_routes(wr, e, mem));
 }
 
-// waves a SIMD that the registers are held to, without spilling but for Q6_K at G = 4 (13). For
+// waves a SIMD that the registers are held to, without spilling but for Q6_K at G = 4 (12). For
 // Q8_0 at G = 1 the rings (70 KB a block) leave two blocks a CU whatever it says
 template <int TYPE, int G>
 constexpr int dm_waves() {
@@ -445,8 +445,8 @@ __global__ __launch_bounds__(DM_THREADS, (dm_waves<TYPE, G>())) void dm_gate_up(
 // to bf16 (the reference's per-route bf16 output), to yv [R, K]. The weighted top-k sum is a
 // launch of its own (dm_combine): inside this one, the blocks of a tile would have to order
 // themselves through device-scope fences, which write back and invalidate the whole L2 of
-// their XCD. The registers are held to 4, 3 and 2 waves a SIMD; Q6_K at NT = 2, G = 4 spills 9 of
-// them for it and IQ3_S at NT = 2, G = 2 three.
+// their XCD. The registers are held to 4, 3 and 2 waves a SIMD; Q6_K at NT = 2, G = 4 spills 11
+// of them for it and IQ3_S at NT = 2, G = 2 four.
 template <int TYPE, int NT, int G, int NR, int NB>
 __global__ __launch_bounds__(DM_THREADS, (G == 1 ? 4 : G == 2 ? 3 : 2)) void dm_down(const uint16_t* __restrict__ hbuf, int K, int N,
                                                       const int32_t* __restrict__ slot_ids, int R, int S,
